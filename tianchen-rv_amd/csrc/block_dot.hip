@@ -114,15 +114,12 @@ __device__ __forceinline__ float2 block_terms(const uint8_t *xc, const uint8_t *
   }
 }
 
-// One wave (64 threads) per pair p.  ncols == 0: x row p, y row p, output
-// s[p].  ncols > 0: x row p / ncols, y row p % ncols, output
-// s[(p / ncols) * bs + p % ncols] (the reference GEMM's loop nest).
+// One wave (64 threads) per pair p: x row p, y row p, output s[p].
 // kSums: write sumi[p*nb + b] instead of the fold.
 template <DotFmt F, bool kSums>
 __global__ __launch_bounds__(64) void block_dot_pairs(size_t nb, float *s, int32_t *sums,
                                                       const uint8_t *vx, size_t bx,
-                                                      const uint8_t *vy, size_t by,
-                                                      size_t ncols, size_t bs) {
+                                                      const uint8_t *vy, size_t by) {
   constexpr int kXBytes = F == DotFmt::kQ8Q8 ? kQ8Bytes : kQ4Bytes;
   // +16: the last even block's 9th dword (or 5th) reads 2 bytes past its end.
   __shared__ __align__(16) uint8_t xl[kChunkBlocks * kXBytes + 16];
@@ -130,14 +127,8 @@ __global__ __launch_bounds__(64) void block_dot_pairs(size_t nb, float *s, int32
   __shared__ float2 terms[kChunkBlocks];
 
   const size_t p = blockIdx.x;
-  size_t xr = p, yr = p, oi = p;
-  if (ncols != 0) {
-    xr = p / ncols;
-    yr = p - xr * ncols;
-    oi = xr * bs + yr;
-  }
-  const uint8_t *xrow = vx + xr * bx;
-  const uint8_t *yrow = vy + yr * by;
+  const uint8_t *xrow = vx + p * bx;
+  const uint8_t *yrow = vy + p * by;
   const int l = threadIdx.x;
   float sumf = 0.0f;
 
@@ -178,7 +169,7 @@ __global__ __launch_bounds__(64) void block_dot_pairs(size_t nb, float *s, int32
   }
   if constexpr (!kSums) {
     if (l == 0)
-      s[oi] = sumf;
+      s[p] = sumf;
   }
 }
 
@@ -410,33 +401,30 @@ int launch_direct_pairs(size_t nb, float *s, size_t os, const uint8_t *vx, size_
 
 template <DotFmt F>
 int launch_pairs(size_t n, float *s, int32_t *sums, const uint8_t *vx, size_t bx,
-                 const uint8_t *vy, size_t by, size_t npairs, size_t ncols, size_t bs,
-                 void *stream) {
+                 const uint8_t *vy, size_t by, size_t npairs, void *stream) {
   const size_t nb = n / tcrv::kQK;
   if (nb == 0 || npairs == 0)
     return TCRV_HIP_OK;  // the reference writes sumf = 0 for nb == 0; see callers
   if (!vx || !vy || (!s && !sums))
     return TCRV_HIP_ERR_NULL_POINTER;
-  const size_t xrows = ncols ? npairs / ncols : npairs;
-  const size_t yrows = ncols ? ncols : npairs;
-  if (!aligned2(vx) || !aligned2(vy) || (xrows > 1 && (bx & 1u)) || (yrows > 1 && (by & 1u)))
+  if (!aligned2(vx) || !aligned2(vy) || (npairs > 1 && ((bx | by) & 1u)))
     return TCRV_HIP_ERR_MISALIGNED;
   const size_t xbytes = nb * (F == DotFmt::kQ8Q8 ? tcrv::kQ8Bytes : tcrv::kQ4Bytes);
-  if ((xrows > 1 && bx < xbytes) || (yrows > 1 && by < nb * tcrv::kQ8Bytes))
+  if (npairs > 1 && (bx < xbytes || by < nb * tcrv::kQ8Bytes))
     return TCRV_HIP_ERR_BAD_SIZE;
   if (npairs > 0x7fffffffu)
     return TCRV_HIP_ERR_TOO_LARGE;
   hipStream_t st = as_stream(stream);
-  const bool direct = !sums && ncols == 0 && nb % 2 == 0 && aligned4(vx) && aligned4(vy) &&
-                      (xrows == 1 || bx % 4 == 0) && (yrows == 1 || by % 4 == 0);
+  const bool direct = !sums && nb % 2 == 0 && aligned4(vx) && aligned4(vy) &&
+                      (npairs == 1 || (bx % 4 == 0 && by % 4 == 0));
   if (direct)
     return launch_direct_pairs<F>(nb, s, 1, vx, bx, vy, by, npairs, st);
   if (sums)
     tcrv::block_dot_pairs<F, true><<<dim3(static_cast<unsigned>(npairs)), dim3(64), 0, st>>>(
-        nb, s, sums, vx, bx, vy, by, ncols, bs);
+        nb, s, sums, vx, bx, vy, by);
   else
     tcrv::block_dot_pairs<F, false><<<dim3(static_cast<unsigned>(npairs)), dim3(64), 0, st>>>(
-        nb, s, sums, vx, bx, vy, by, ncols, bs);
+        nb, s, sums, vx, bx, vy, by);
   return launch_status();
 }
 
@@ -489,16 +477,6 @@ int q4_0_rows_direct(size_t nb, float *s, size_t os, const uint8_t *vx, size_t b
   return rows_direct<DotFmt::kQ4Q8>(nb, s, os, vx, bx, vy, by, npairs, stream);
 }
 
-int q4_0_grid(size_t n, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by,
-              size_t nr, size_t nc, size_t bs, void *stream) {
-  if (n / tcrv::kQK == 0)
-    return zero_outputs(s, nr * nc, bs, nc, stream);
-  if (!s)
-    return TCRV_HIP_ERR_NULL_POINTER;
-  return launch_pairs<tcrv::DotFmt::kQ4Q8>(n, s, nullptr, vx, bx, vy, by, nr * nc, nc, bs,
-                                           stream);
-}
-
 }  // namespace tcrv_host
 
 using tcrv_host::zero_outputs;
@@ -511,8 +489,7 @@ int tcrv_hip_q8_0_q8_0_block_dot(size_t n, float *s, const uint8_t *vx, const ui
     return zero_outputs(s, 1, 0, 0, stream);
   if (!s)
     return TCRV_HIP_ERR_NULL_POINTER;
-  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ8Q8>(n, s, nullptr, vx, 0, vy, 0, 1, 0, 0,
-                                                      stream);
+  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ8Q8>(n, s, nullptr, vx, 0, vy, 0, 1, stream);
 }
 
 int tcrv_hip_q8_0_q8_0_block_dot_rows(size_t n, float *s, const uint8_t *vx, size_t bx,
@@ -522,8 +499,7 @@ int tcrv_hip_q8_0_q8_0_block_dot_rows(size_t n, float *s, const uint8_t *vx, siz
     return zero_outputs(s, nrows, 0, 0, stream);
   if (!s)
     return TCRV_HIP_ERR_NULL_POINTER;
-  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ8Q8>(n, s, nullptr, vx, bx, vy, by, nrows,
-                                                      0, 0, stream);
+  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ8Q8>(n, s, nullptr, vx, bx, vy, by, nrows, stream);
 }
 
 int tcrv_hip_q4_0_q8_0_block_dot(size_t n, float *s, size_t bs, const uint8_t *vx,
@@ -537,8 +513,7 @@ int tcrv_hip_q4_0_q8_0_block_dot(size_t n, float *s, size_t bs, const uint8_t *v
     return zero_outputs(s, 1, 0, 0, stream);
   if (!s)
     return TCRV_HIP_ERR_NULL_POINTER;
-  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ4Q8>(n, s, nullptr, vx, 0, vy, 0, 1, 0, 0,
-                                                      stream);
+  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ4Q8>(n, s, nullptr, vx, 0, vy, 0, 1, stream);
 }
 
 int tcrv_hip_q4_0_q8_0_block_dot_rows(size_t n, float *s, const uint8_t *vx, size_t bx,
@@ -548,8 +523,7 @@ int tcrv_hip_q4_0_q8_0_block_dot_rows(size_t n, float *s, const uint8_t *vx, siz
     return zero_outputs(s, nrows, 0, 0, stream);
   if (!s)
     return TCRV_HIP_ERR_NULL_POINTER;
-  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ4Q8>(n, s, nullptr, vx, bx, vy, by, nrows,
-                                                      0, 0, stream);
+  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ4Q8>(n, s, nullptr, vx, bx, vy, by, nrows, stream);
 }
 
 int tcrv_hip_q8_0_q8_0_block_sums(size_t n, int32_t *sumi, const uint8_t *vx, size_t bx,
@@ -558,8 +532,7 @@ int tcrv_hip_q8_0_q8_0_block_sums(size_t n, int32_t *sumi, const uint8_t *vx, si
     return TCRV_HIP_OK;
   if (!sumi)
     return TCRV_HIP_ERR_NULL_POINTER;
-  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ8Q8>(n, nullptr, sumi, vx, bx, vy, by, nrows,
-                                                      0, 0, stream);
+  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ8Q8>(n, nullptr, sumi, vx, bx, vy, by, nrows, stream);
 }
 
 int tcrv_hip_q4_0_q8_0_block_sums(size_t n, int32_t *sumi, const uint8_t *vx, size_t bx,
@@ -568,8 +541,7 @@ int tcrv_hip_q4_0_q8_0_block_sums(size_t n, int32_t *sumi, const uint8_t *vx, si
     return TCRV_HIP_OK;
   if (!sumi)
     return TCRV_HIP_ERR_NULL_POINTER;
-  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ4Q8>(n, nullptr, sumi, vx, bx, vy, by, nrows,
-                                                      0, 0, stream);
+  return tcrv_host::launch_pairs<tcrv::DotFmt::kQ4Q8>(n, nullptr, sumi, vx, bx, vy, by, nrows, stream);
 }
 
 }  // extern "C"

@@ -1821,6 +1821,14 @@ bool ws_rows_few_first(size_t nb, const uint8_t *vx, size_t bx, const uint8_t *v
          !tiles16_first(nr, nc) && tiles64_of(nr, nc) <= 448;
 }
 
+// Shapes that take a workspace by the rule below but do not need it: few tokens,
+// where gemm_batch reads the plain rows faster than they are packed (us, K 4096,
+// Q4_0 / Q8_0, against pack and tiles: 4096 x 32 10.0 / 11.0 against 27 / 24).
+// The workspace is checked all the same and left untouched.
+bool ws_batch_first(size_t nr, size_t nc) {
+  return nc <= 16 || (nc <= 64 && (nr + 15) / 16 * ((nc + 15) / 16) <= 1024);
+}
+
 bool gemm_ws_uses_workspace(size_t n, const uint8_t *vx, size_t bx, const uint8_t *vy,
                             size_t by, size_t nr, size_t nc) {
   const size_t nb = n / tcrv::kQK;
@@ -1857,6 +1865,8 @@ int tcrv_hip_q8_0_q8_0_gemm_ws(size_t n, float *s, const uint8_t *vx, const uint
   const size_t tx_bytes = tile_bytes(nr, nb), ty_bytes = tile_bytes(nc, nb);
   if (workspace_bytes < tx_bytes + ty_bytes)
     return TCRV_HIP_ERR_BAD_SIZE;
+  if (ws_batch_first(nr, nc))
+    return gemm_batch(false, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
   uint8_t *tx = static_cast<uint8_t *>(workspace);
   uint8_t *ty = tx + tx_bytes;  // tx_bytes is a multiple of 2176 = 16 * 136
   hipStream_t st = as_stream(stream);
@@ -1920,6 +1930,8 @@ int tcrv_hip_q4_0_q8_0_gemm_ws(size_t n, float *s, const uint8_t *vx, const uint
   const size_t tx_bytes = tile_bytes(nr, nb), ty_bytes = tile_bytes(nc, nb);
   if (workspace_bytes < tx_bytes + ty_bytes)
     return TCRV_HIP_ERR_BAD_SIZE;
+  if (ws_batch_first(nr, nc))
+    return gemm_batch(true, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
   uint8_t *tx = static_cast<uint8_t *>(workspace);
   uint8_t *ty = tx + tx_bytes;  // tx_bytes is a multiple of 2176 = 16 * 136
   hipStream_t st = as_stream(stream);

@@ -172,8 +172,7 @@ inline hipStream_t as_stream(void *stream) { return reinterpret_cast<hipStream_t
 // s[(i / ncols) * stride + i % ncols] (what the reference writes when nb == 0).
 int zero_outputs(float *s, size_t count, size_t stride, size_t ncols, void *stream);
 
-// Q4_0 x Q8_0 GEMM for nc > 1 on MFMA (gemm.hip); TCRV_HIP_ERR_UNSUPPORTED when
-// rows are not 4-byte aligned.
+// Q4_0 x Q8_0 GEMM for nc > 1 on MFMA, rows 4-byte aligned (gemm.hip).
 int q4_0_gemm_mfma(size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
                    size_t by, size_t nr, size_t nc, size_t bs, void *stream);
 
@@ -186,9 +185,28 @@ int q8_0_rows_direct(size_t nb, float *s, size_t os, const uint8_t *vx, size_t b
 int q4_0_rows_direct(size_t nb, float *s, size_t os, const uint8_t *vx, size_t bx,
                      const uint8_t *vy, size_t by, size_t npairs, void *stream);
 
-// Q4_0 x Q8_0 GEMM for nc > 1 as one wave per output element (block_dot.hip).
-int q4_0_grid(size_t n, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by,
-              size_t nr, size_t nc, size_t bs, void *stream);
+// The GEMMs over 16 x 16 tiles with K split over a work-group's waves
+// (gemm_batch.hip): any 2-byte aligned rows, any block count, any nr and nc.
+int gemm_batch(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
+               size_t by, size_t nr, size_t nc, size_t bs, void *stream);
+// Whether it runs a shape first (rows4: rows and strides 4-byte aligned).
+//   - Rows that are not: always (the other kernels need dwords).
+//   - From 5 tokens: up to 24 always, up to 64 while its work-groups fit two
+//     rounds of two a CU (us, K 4096, Q4_0 / Q8_0 against the kernel that ran
+//     before: 4096 x 5 6.4 / 7.1 against 8.2 / 8.9, 14336 x 8 17.2 / 19.2
+//     against 28.7 / 29.1, 4096 x 64 16.8 / 18.2 against 30.8 / 26.4; past the
+//     bound 14336 x 64 53 / 56 against 31.6 / 27.5).
+//   - Up to 4 tokens the multi-column GEMVs where they serve the rows (even
+//     block count; 4096 x 4 4.9 / 6.8 against 6.4 / 7.1), but 3 and 4 at K up to
+//     2048, one of its chunks (2048 x 4 x 2048 4.2 / 4.2 against 4.5 / 5.1, 14336 x 4 x
+//     1024 7.1 / 7.9 against 9.1 / 11.3; at K 2944 5.8 / 6.2 against 4.8 / 5.9).
+inline bool batch_first(bool rows4, size_t nb, size_t nr, size_t nc) {
+  if (!rows4)
+    return true;
+  if (nc <= 4 && nb % 2 == 0)
+    return nr > 1 && nc >= 3 && nb <= 64;
+  return nc <= 24 || (nc <= 64 && (nr + 15) / 16 * ((nc + 15) / 16) <= 1024);
+}
 
 // The GEMMs with 2..kGemvColsMax tokens (batched decode) run as multi-column
 // GEMVs over groups of up to eight activation columns, the weights read once
