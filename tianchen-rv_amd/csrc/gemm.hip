@@ -793,19 +793,20 @@ extern "C" int tcrv_hip_q8_0_q8_0_gemm(size_t n, float *s, const uint8_t *vx,
   }
   const bool rows4 = aligned4(vx) && aligned4(vy) && (nr == 1 || bx % 4 == 0) &&
                      (nc == 1 || by % 4 == 0);
-  if (batch_first(rows4, nb, nr, nc))
-    return gemm_batch(false, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
-  if (nc > 1 && nr > 1) {
-    if (!cols_first(nr, nc)) {  // few output tiles: one 32 x 32 tile a wave
-      const int st = gemm_rows_few(false, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
-      if (st != TCRV_HIP_ERR_UNSUPPORTED)
-        return st;
-    }
-    if (nc <= kGemvColsMax) {  // a few tokens: multi-column GEMVs
-      const int st = gemv_cols_q8_0_q8_0(nb, s, bs, vx, bx, vy, by, nr, nc, stream);
-      if (st != TCRV_HIP_ERR_UNSUPPORTED)
-        return st;
-    }
+  {
+    const int st = gemm_small(false, rows4, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
+    if (st != TCRV_HIP_ERR_UNSUPPORTED)
+      return st;
+  }
+  if (nc <= kGemvColsMax) {  // a few tokens: one multi-column GEMV
+    const int st = gemv_cols_q8_0_q8_0(nb, s, bs, vx, bx, vy, by, nr, nc, stream);
+    if (st != TCRV_HIP_ERR_UNSUPPORTED)
+      return st;
+  }
+  {  // few output tiles: one 32 x 32 tile a wave
+    const int st = gemm_rows_few(false, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
+    if (st != TCRV_HIP_ERR_UNSUPPORTED)
+      return st;
   }
   const size_t tiles =
       ((nr + tcrv::kFbBM - 1) / tcrv::kFbBM) * ((nc + tcrv::kFbBN - 1) / tcrv::kFbBN);

@@ -1779,14 +1779,18 @@ namespace tcrv_host {
 // rows 16-byte aligned, a whole number of 8-block chunks, the shapes
 // gemm_tiles32 serves (at its 1024 work-groups the 256-row kernels are as fast:
 // 4096 x 1024 x 4096 Q8_0 91.6 against 91-93 us).
+bool rows_few_serves(size_t nb, const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by,
+                     size_t nr, size_t nc) {
+  return nr >= 2 && nc >= 2 && nb != 0 && nb % tcrv::kFKB == 0 && aligned16(vx) &&
+         aligned16(vy) && bx % 16 == 0 && by % 16 == 0 &&
+         tiles32_first(tiles128_of(nr, nc), tiles64_of(nr, nc), nb);
+}
+
 int gemm_rows_few(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
                   size_t by, size_t nr, size_t nc, size_t bs, void *stream) {
-  if (nr < 2 || nc < 2 || nb == 0 || nb % tcrv::kFKB != 0 || !aligned16(vx) || !aligned16(vy) ||
-      bx % 16 != 0 || by % 16 != 0)
+  if (!rows_few_serves(nb, vx, bx, vy, by, nr, nc))
     return TCRV_HIP_ERR_UNSUPPORTED;
   const size_t tiles64 = tiles64_of(nr, nc);
-  if (!tiles32_first(tiles128_of(nr, nc), tiles64, nb))
-    return TCRV_HIP_ERR_UNSUPPORTED;
   const dim3 g(static_cast<unsigned>(tiles64)), b(256);
   const unsigned nbu = static_cast<unsigned>(nb);
   if (q4)
@@ -1796,18 +1800,15 @@ int gemm_rows_few(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, co
   return launch_status();
 }
 
+// Which calls take a workspace (and are refused without one) is part of the entries'
+// contract; which kernel then runs is not.
 // Shapes the tiled kernel does not serve run as tcrv_hip_q8_0_q8_0_gemm,
 // without the workspace: fewer weight rows than one 256-row tile, a single
-// token (decode), no blocks, or more than kMaxTiledNb blocks.  So do a few
-// tokens that the plain entry's multi-column GEMVs take (even block count,
-// 4-byte aligned rows and strides; cols_first): there they beat packing both
-// operands for the tiled kernels (us, 4096 weight rows, K 4096, Q8_0 / Q4_0:
-// 16 tokens 15.0 / 16.3 against ~25 / ~28; 32 tokens 30.8 / 32.3 against
-// 23.9 / 26.9).
-bool ws_cols_first(size_t nb, const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by,
-                   size_t nr, size_t nc) {
-  return cols_first(nr, nc) && nb % 2 == 0 && aligned4(vx) && aligned4(vy) && bx % 4 == 0 &&
-         by % 4 == 0;
+// token (decode), no blocks, or more than kMaxTiledNb blocks.  So do up to 24
+// tokens over an even block count and 4-byte aligned rows and strides.
+bool ws_few_tokens(size_t nb, const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by,
+                   size_t nc) {
+  return nc <= 24 && nb % 2 == 0 && aligned4(vx) && aligned4(vy) && bx % 4 == 0 && by % 4 == 0;
 }
 // And where the plain entry's few-tile kernel, which packs in LDS, beats a
 // separate pack: up to 448 of its work-groups at K up to 4096, past the 16 x 16
@@ -1821,19 +1822,30 @@ bool ws_rows_few_first(size_t nb, const uint8_t *vx, size_t bx, const uint8_t *v
          !tiles16_first(nr, nc) && tiles64_of(nr, nc) <= 448;
 }
 
-// Shapes that take a workspace by the rule below but do not need it: few tokens,
-// where gemm_batch reads the plain rows faster than they are packed (us, K 4096,
-// Q4_0 / Q8_0, against pack and tiles: 4096 x 32 10.0 / 11.0 against 27 / 24).
-// The workspace is checked all the same and left untouched.
-bool ws_batch_first(size_t nr, size_t nc) {
-  return nc <= 16 || (nc <= 64 && (nr + 15) / 16 * ((nc + 15) / 16) <= 1024);
+// Shapes that take a workspace by the rule below but do not need it: few outputs,
+// where gemm_batch and gemm_rows16 read the plain rows faster than they are packed (us, K
+// 4096, Q4_0 / Q8_0, against pack and tiles: 4096 x 32 10.0 / 11.0 against 27 / 24,
+// 14336 x 200 x 2048 57 / 51 against 70 / 62, 3001 x 100 x 2912 15.7 / 16.2 against 24.1
+// / 22.9; past 256 64-row work-groups the tiles win, 4096 x 256 x 4160 33.8 / 35.8
+// against 33.2 / 30.3).  The workspace is checked all the same and left untouched.
+bool ws_small_first(size_t nr, size_t nc) {
+  return nc <= 16 || (nr + 15) / 16 * ((nc + 15) / 16) <= 512 ||
+         (nr + 63) / 64 * ((nc + 31) / 32) <= 256;
+}
+int ws_small(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
+             size_t by, size_t nr, size_t nc, size_t bs, void *stream) {
+  if (!ws_small_first(nr, nc))
+    return TCRV_HIP_ERR_UNSUPPORTED;
+  if (nc <= 16 || (nr + 15) / 16 * ((nc + 15) / 16) <= 512)
+    return gemm_batch(q4, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
+  return gemm_rows16(q4, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
 }
 
 bool gemm_ws_uses_workspace(size_t n, const uint8_t *vx, size_t bx, const uint8_t *vy,
                             size_t by, size_t nr, size_t nc) {
   const size_t nb = n / tcrv::kQK;
   return nr >= static_cast<size_t>(tcrv::kDBM) && nc >= 2 && nb > 0 && nb <= kMaxTiledNb &&
-         !ws_cols_first(nb, vx, bx, vy, by, nr, nc) &&
+         !ws_few_tokens(nb, vx, bx, vy, by, nc) &&
          !ws_rows_few_first(nb, vx, bx, vy, by, nr, nc);
 }
 
@@ -1865,8 +1877,11 @@ int tcrv_hip_q8_0_q8_0_gemm_ws(size_t n, float *s, const uint8_t *vx, const uint
   const size_t tx_bytes = tile_bytes(nr, nb), ty_bytes = tile_bytes(nc, nb);
   if (workspace_bytes < tx_bytes + ty_bytes)
     return TCRV_HIP_ERR_BAD_SIZE;
-  if (ws_batch_first(nr, nc))
-    return gemm_batch(false, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
+  {
+    const int rc = ws_small(false, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
+    if (rc != TCRV_HIP_ERR_UNSUPPORTED)
+      return rc;
+  }
   uint8_t *tx = static_cast<uint8_t *>(workspace);
   uint8_t *ty = tx + tx_bytes;  // tx_bytes is a multiple of 2176 = 16 * 136
   hipStream_t st = as_stream(stream);
@@ -1930,8 +1945,11 @@ int tcrv_hip_q4_0_q8_0_gemm_ws(size_t n, float *s, const uint8_t *vx, const uint
   const size_t tx_bytes = tile_bytes(nr, nb), ty_bytes = tile_bytes(nc, nb);
   if (workspace_bytes < tx_bytes + ty_bytes)
     return TCRV_HIP_ERR_BAD_SIZE;
-  if (ws_batch_first(nr, nc))
-    return gemm_batch(true, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
+  {
+    const int rc = ws_small(true, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
+    if (rc != TCRV_HIP_ERR_UNSUPPORTED)
+      return rc;
+  }
   uint8_t *tx = static_cast<uint8_t *>(workspace);
   uint8_t *ty = tx + tx_bytes;  // tx_bytes is a multiple of 2176 = 16 * 136
   hipStream_t st = as_stream(stream);

@@ -374,7 +374,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemv_q4_0_q8_0_half(float *s, siz
 }
 
 // Multi-column form of the register-direct GEMV, for the a7 GEMM with a few
-// tokens (batched decode, nc = 2..kGemvColsMax): each wave loads its 4 weight
+// tokens (batched decode, nc = 2..4): each wave loads its 4 weight
 // rows' block pairs once and dots them with kCols activation columns (ncols of
 // them present; absent ones re-read the last and are not stored).  Per (row,
 // column) the terms fl((float)sumi * d_x) and the column's d_y go through the
@@ -387,9 +387,9 @@ __global__ __launch_bounds__(256) void gemv_q4_0_q8_0_cols(size_t nb_arg, float 
                                                            size_t nr, int ncols) {
   constexpr int kWaves = 4, kR = 4;
   constexpr int kChains = kR * kCols;
-  constexpr int kLanes = 64 / kChains;       // 8 lanes for 2 columns, 4 for 4, 2 for 8
+  constexpr int kLanes = 64 / kChains;       // 8 lanes for 2 columns, 4 for 4
   constexpr int kTerms = kGvChunk / kLanes;  // blocks per fold lane
-  static_assert(kLanes == 8 || kLanes == 4 || kLanes == 2, "fold groups inside one DPP row");
+  static_assert(kLanes == 8 || kLanes == 4, "fold groups inside one DPP row");
   const size_t nb = kOneChunk ? static_cast<size_t>(kGvChunk) : nb_arg;
   __shared__ __align__(16) float tl[kWaves][kChains][kGvChunk + 4];
   __shared__ __align__(16) float dyl[kWaves][kCols][kGvChunk];
@@ -510,9 +510,9 @@ __global__ __launch_bounds__(256) void gemv_q8_0_q8_0_cols(size_t nb_arg, float 
                                                            size_t nr, int ncols) {
   constexpr int kWaves = 4, kR = 4;
   constexpr int kChains = kR * kCols;
-  constexpr int kLanes = 64 / kChains;       // 8 lanes for 2 columns, 4 for 4, 2 for 8
+  constexpr int kLanes = 64 / kChains;       // 8 lanes for 2 columns, 4 for 4
   constexpr int kTerms = kGvChunk / kLanes;  // blocks per fold lane
-  static_assert(kLanes == 8 || kLanes == 4 || kLanes == 2, "fold groups inside one DPP row");
+  static_assert(kLanes == 8 || kLanes == 4, "fold groups inside one DPP row");
   const size_t nb = kOneChunk ? static_cast<size_t>(kGvChunk) : nb_arg;
   __shared__ __align__(16) float2 tl[kWaves][kChains][kGvChunk + 2];  // ((float)sumi, d_x*d_y)
 
@@ -678,37 +678,16 @@ int launch_cols(size_t nb, float *s, size_t bs, const uint8_t *vx, size_t bx, co
   return launch_status();
 }
 
-// Columns in groups: eight while five or more are left (five to seven present
-// in the last), then four (three or four present), two, and a single column
-// through the decode GEMV (Q4_0) or the block dots (Q8_0).
 template <bool kQ4>
 int gemv_cols(size_t nb, float *s, size_t bs, const uint8_t *vx, size_t bx, const uint8_t *vy,
               size_t by, size_t nr, size_t nc, void *stream) {
-  if (nb % 2 != 0 || !aligned4(vx) || !aligned4(vy) || (nr > 1 && bx % 4 != 0) || by % 4 != 0)
+  if (nb % 2 != 0 || !aligned4(vx) || !aligned4(vy) || (nr > 1 && bx % 4 != 0) || by % 4 != 0 ||
+      nc < 2 || nc > kGemvColsMax)
     return TCRV_HIP_ERR_UNSUPPORTED;
   hipStream_t st = as_stream(stream);
-  for (size_t c0 = 0; c0 < nc;) {
-    const size_t rem = nc - c0;
-    float *sc = s + c0;
-    const uint8_t *yc = vy + c0 * by;
-    const size_t take = rem >= 5 ? (rem < 8 ? rem : 8) : rem;  // rem <= 4: one last group
-    int rc;
-    if (rem >= 5)
-      rc = launch_cols<kQ4, 8>(nb, sc, bs, vx, bx, yc, by, nr, static_cast<int>(take), st);
-    else if (rem >= 3)
-      rc = launch_cols<kQ4, 4>(nb, sc, bs, vx, bx, yc, by, nr, static_cast<int>(take), st);
-    else if (rem == 2)
-      rc = launch_cols<kQ4, 2>(nb, sc, bs, vx, bx, yc, by, nr, 2, st);
-    else if constexpr (kQ4)
-      rc = nr <= kDirectSmallRows ? launch_direct<2>(nb, sc, bs, vx, bx, yc, nr, st)
-                                  : launch_direct<kDirectRows>(nb, sc, bs, vx, bx, yc, nr, st);
-    else
-      rc = q8_0_rows_direct(nb, sc, bs, vx, bx, yc, 0, nr, stream);
-    if (rc != TCRV_HIP_OK)
-      return rc;
-    c0 += take;
-  }
-  return TCRV_HIP_OK;
+  if (nc == 2)
+    return launch_cols<kQ4, 2>(nb, s, bs, vx, bx, vy, by, nr, 2, st);
+  return launch_cols<kQ4, 4>(nb, s, bs, vx, bx, vy, by, nr, static_cast<int>(nc), st);
 }
 
 int gemv_cols_q4_0_q8_0(size_t nb, float *s, size_t bs, const uint8_t *vx, size_t bx,
@@ -843,21 +822,22 @@ int tcrv_hip_q4_0_q8_0_gemm(size_t n, float *s, const uint8_t *vx, const uint8_t
   }
   const bool rows4 = tcrv_host::aligned4(vx) && tcrv_host::aligned4(vy) &&
                      (nr == 1 || bx % 4 == 0) && by % 4 == 0;
-  if (tcrv_host::batch_first(rows4, nb, nr, nc))
-    return tcrv_host::gemm_batch(true, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
-  if (nr > 1) {
-    if (!tcrv_host::cols_first(nr, nc)) {  // few output tiles: one 32 x 32 tile a wave
-      const int st = tcrv_host::gemm_rows_few(true, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
-      if (st != TCRV_HIP_ERR_UNSUPPORTED)
-        return st;
-    }
-    if (nc <= tcrv_host::kGemvColsMax) {
-      // a few tokens: the weights are read once per group of up to eight
-      // columns (the MFMA GEMM would run only nr / 256 work-groups)
-      const int st = tcrv_host::gemv_cols_q4_0_q8_0(nb, s, bs, vx, bx, vy, by, nr, nc, stream);
-      if (st != TCRV_HIP_ERR_UNSUPPORTED)
-        return st;
-    }
+  {
+    const int st = tcrv_host::gemm_small(true, rows4, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
+    if (st != TCRV_HIP_ERR_UNSUPPORTED)
+      return st;
+  }
+  if (nc <= tcrv_host::kGemvColsMax) {
+    // a few tokens: the weights are read once for all columns (the MFMA GEMM
+    // would run only nr / 256 work-groups)
+    const int st = tcrv_host::gemv_cols_q4_0_q8_0(nb, s, bs, vx, bx, vy, by, nr, nc, stream);
+    if (st != TCRV_HIP_ERR_UNSUPPORTED)
+      return st;
+  }
+  {  // few output tiles: one 32 x 32 tile a wave
+    const int st = tcrv_host::gemm_rows_few(true, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
+    if (st != TCRV_HIP_ERR_UNSUPPORTED)
+      return st;
   }
   return tcrv_host::q4_0_gemm_mfma(nb, s, vx, bx, vy, by, nr, nc, bs, stream);
 }

@@ -190,43 +190,48 @@ int q4_0_rows_direct(size_t nb, float *s, size_t os, const uint8_t *vx, size_t b
 int gemm_batch(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
                size_t by, size_t nr, size_t nc, size_t bs, void *stream);
 // Whether it runs a shape first (rows4: rows and strides 4-byte aligned).
-//   - Rows that are not: always (the other kernels need dwords).
-//   - From 5 tokens: up to 24 always, up to 64 while its work-groups fit two
-//     rounds of two a CU (us, K 4096, Q4_0 / Q8_0 against the kernel that ran
-//     before: 4096 x 5 6.4 / 7.1 against 8.2 / 8.9, 14336 x 8 17.2 / 19.2
-//     against 28.7 / 29.1, 4096 x 64 16.8 / 18.2 against 30.8 / 26.4; past the
-//     bound 14336 x 64 53 / 56 against 31.6 / 27.5).
+//   - Up to 16 tokens from 5 (us, K 4096, Q4_0 / Q8_0, against the multi-column
+//     GEMVs: 4096 x 5 6.4 / 7.1 against 8.2 / 8.9, 14336 x 8 17.2 / 19.2 against 28.7 /
+//     29.1), and up to 16 weight rows; past that while its work-groups fit one round of two
+//     a CU, whatever the tokens (2048 x 64 10.1 / 11.0 against 12.3 / 11.8 of gemm_rows16,
+//     512 x 200 10.0 / 10.6 against 12.4 / 11.9; 4096 x 64, two rounds, 18.0 / 18.7 against
+//     13.4 / 12.4).
 //   - Up to 4 tokens the multi-column GEMVs where they serve the rows (even
 //     block count; 4096 x 4 4.9 / 6.8 against 6.4 / 7.1), but 3 and 4 at K up to
 //     2048, one of its chunks (2048 x 4 x 2048 4.2 / 4.2 against 4.5 / 5.1, 14336 x 4 x
 //     1024 7.1 / 7.9 against 9.1 / 11.3; at K 2944 5.8 / 6.2 against 4.8 / 5.9).
 inline bool batch_first(bool rows4, size_t nb, size_t nr, size_t nc) {
-  if (!rows4)
-    return true;
-  if (nc <= 4 && nb % 2 == 0)
+  if (rows4 && nc <= 4 && nb % 2 == 0)
     return nr > 1 && nc >= 3 && nb <= 64;
-  return nc <= 24 || (nc <= 64 && (nr + 15) / 16 * ((nc + 15) / 16) <= 1024);
+  return nc <= 16 || nr <= 16 || (nr + 15) / 16 * ((nc + 15) / 16) <= 512;
 }
 
-// The GEMMs with 2..kGemvColsMax tokens (batched decode) run as multi-column
-// GEMVs over groups of up to eight activation columns, the weights read once
-// per group (gemv.hip); an MFMA GEMM would run only nr / 256 work-groups.
-// TCRV_HIP_ERR_UNSUPPORTED for an odd block count or operands/strides that are
-// not 4-byte aligned.
-constexpr size_t kGemvColsMax = 64;
-// The multi-column GEMVs run first up to kColsFirstMax tokens; past it the
-// one-tile-a-wave GEMMs (gemm_rows_few from plain rows, gemm_tiled.hip) where
-// they serve the shape, then the GEMVs up to kGemvColsMax.  A GEMV launch
-// serves 8 tokens at ~6 us for K 4096 whatever the weight rows (it is bound by
-// its K loop at few rows: 256 x 40 x 4096 Q8_0 32 us as five launches against
-// 18-27 us on the tiles), so the switch depends on the tokens only.
-constexpr size_t kColsFirstMax = 24;
-inline bool cols_first(size_t nr, size_t nc) {
-  (void)nr;
-  return nc <= kColsFirstMax;
-}
-// The GEMM of few output tiles straight from plain rows (16-byte aligned rows
-// and strides, n a multiple of 256); TCRV_HIP_ERR_UNSUPPORTED otherwise.
+// The GEMMs with one 16 x 16 tile a wave, a work-group's rows shared through LDS
+// (gemm_rows16.hip): any 2-byte aligned rows, any block count.
+// TCRV_HIP_ERR_UNSUPPORTED for row strides past 64 MB (and over 2 million tokens
+// or 16 million rows).
+int gemm_rows16(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
+                size_t by, size_t nr, size_t nc, size_t bs, void *stream);
+
+// The plain-row GEMMs of few outputs and those of rows that are not 4-byte aligned:
+// gemm_batch or gemm_rows16, or TCRV_HIP_ERR_UNSUPPORTED where the kernels for
+// 4-byte aligned rows are faster (the multi-column GEMVs; gemm_rows_few past three
+// rounds of 32-row work-groups: 4096 x 192 x 4096 31.2 / 26.8 against 28.1 / 26.0
+// us, 4096 x 256 31.4 / 27.0 against 29.9 / 31.6; where it does not serve the rows,
+// the 256-row tiles past 1024 64-row work-groups: K 4160, 4096 x 512 101 / 93.6
+// against 61 / 70, 4096 x 1000 101 / 92.5 against 118 / 138).
+int gemm_small(bool q4, bool rows4, size_t nb, float *s, const uint8_t *vx, size_t bx,
+               const uint8_t *vy, size_t by, size_t nr, size_t nc, size_t bs, void *stream);
+
+// The GEMMs with 2 to 4 tokens as one multi-column GEMV launch, the weights read
+// once (gemv.hip).  TCRV_HIP_ERR_UNSUPPORTED for more tokens, an odd block count or
+// operands/strides that are not 4-byte aligned.
+constexpr size_t kGemvColsMax = 4;
+// The GEMM of few output tiles straight from plain rows (gemm_tiled.hip): rows 16-byte
+// aligned, n a multiple of 256, at most 1024 work-groups of 64 x 64.
+bool rows_few_serves(size_t nb, const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by,
+                     size_t nr, size_t nc);
+// TCRV_HIP_ERR_UNSUPPORTED where it does not serve.
 int gemm_rows_few(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
                   size_t by, size_t nr, size_t nc, size_t bs, void *stream);
 int gemv_cols_q4_0_q8_0(size_t nb, float *s, size_t bs, const uint8_t *vx, size_t bx,
