@@ -83,7 +83,9 @@ __device__ __forceinline__ BtPair bt_q8_pair_for_q4(const uint32_t *w, int k) {
 
 // A Q4_0 pair (9 dwords): the same byte positions, the nibbles as 16 (n - 8) --
 // the offset-binary nibble with its top bit flipped, left in the byte's high
-// half, so the sums are 16 sumi and d_x is used as d_x / 16 (both exact).
+// half.  Sums, terms and the running fold are then 16 times the reference's, exactly (a power
+// of two, and nothing comes near either end of the exponent range: terms are
+// multiples of 2^-48 below 2^47), and the stored value is acc / 16.
 __device__ __forceinline__ BtPair bt_q4_pair(const uint32_t *w, int k) {
   BtPair p;
   const uint32_t z = w[0], a = w[1 + k];
@@ -216,7 +218,7 @@ __global__ __launch_bounds__(kWaves * 64, 4) void gemm_batch(
   auto step = [&](float fs, uint32_t dx, uint32_t dy) {
     const float x = fp16_bits_to_f32(dx), y = fp16_bits_to_f32(dy);
     if constexpr (kQ4)
-      acc = fmaf(fs * fmaf(x, 0.0625f, -0.0f), y, acc);
+      acc = fmaf(fmaf(fs, x, -0.0f), y, acc);
     else
       acc = fmaf(fs, fmaf(x, y, -0.0f), acc);
   };
@@ -305,7 +307,7 @@ __global__ __launch_bounds__(kWaves * 64, 4) void gemm_batch(
     __syncthreads();
   }
   if (wave < 4 && row0 + fr < nr && li < ntok)
-    s[(row0 + fr) * bs + tok0 + li] = acc;
+    s[(row0 + fr) * bs + tok0 + li] = kQ4 ? acc * 0.0625f : acc;
 }
 
 }  // namespace tcrv
