@@ -239,6 +239,11 @@ int gemv_cols_q4_0_q8_0(size_t nb, float *s, size_t bs, const uint8_t *vx, size_
 int gemv_cols_q8_0_q8_0(size_t nb, float *s, size_t bs, const uint8_t *vx, size_t bx,
                         const uint8_t *vy, size_t by, size_t nr, size_t nc, void *stream);
 
+// The x16 repack GEMM on 64- or 128-row work-groups (gemm_repack.hip), or
+// TCRV_HIP_ERR_UNSUPPORTED where wide_tiles work-groups of 256 x 128 are faster.
+int gemm_repack_mid(size_t nb, float *s, const uint8_t *vx, const uint8_t *vy, size_t ngw,
+                    size_t nga, size_t bs, bool vec_out, size_t wide_tiles, void *stream);
+
 // tcrv_hip_q8_0_q8_0_gemm_ws packs into its workspace and runs the tiled
 // kernels for this call (otherwise it runs the plain GEMM and reads no
 // workspace); gemm_tiled.hip.
