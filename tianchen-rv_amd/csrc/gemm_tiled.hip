@@ -710,7 +710,7 @@ static_assert(kEStages * (kEStage + kEKB * kEHRow * 2) <= 160 * 1024,
 static_assert(kEKB <= 4, "the scale moves of a chunk are waves 0-3's");
 
 // kQ4: the weight groups hold Q4_0 rows decoded to int8 (as gemm_tiles_q4's)
-// and the fold is the Q4_0 one on transposed tiles (fold_chunk_q4_2x4): the
+// and the fold is the Q4_0 one on transposed tiles (fold_chunk_q4_tiles): the
 // waves that move a block's scales (waves 0-3, block w) also widen its 256
 // token scales to the fp32 row fyd before the barrier that publishes the
 // chunk, the fast fold runs until a chunk holds a non-finite d_x among the
@@ -769,10 +769,24 @@ __device__ __forceinline__ void global_load_lds_asm(const uint8_t *from, lds_voi
                : "memory");
 }
 
-// One wave's view of a 256 x 256 work-group: its tile, its DMA slots and the
+// Wave tiles of a work-group: 4 x 2 waves of 2 x 4 tiles (256 x 256 outputs) or 2 x 4
+// waves of 3 x 2 tiles (192 x 256).  The smaller one keeps the larger one's LDS and DMA
+// layout with the fourth weight group left out.
+struct Wave2x4 {
+  static constexpr int kNI = 2, kNJ = 4, kWaveRows = 4;
+};
+struct Wave3x2 {
+  static constexpr int kNI = 3, kNJ = 2, kWaveRows = 2;
+};
+
+// One wave's view of a work-group: its tile, its DMA slots and the
 // LDS operands of its lanes.
+template <typename W>
 struct Tiles256 {
-  int wave, lane, wm, wn, li, h;  // wm, wn: 64 weight rows x 128 tokens per wave
+  static constexpr int kRows = 32 * W::kNI, kToks = 32 * W::kNJ;  // of a wave
+  static constexpr int kBM = kRows * W::kWaveRows;
+  static_assert(kToks * (8 / W::kWaveRows) == kEBN && kBM % kTG == 0, "whole groups");
+  int wave, lane, wm, wn, li, h;  // wm, wn: kRows weight rows x kToks tokens per wave
   size_t m0, n0, nb, nchunks;
   const uint8_t *own;  // the wave's row group's records (wave-uniform)
   const uint8_t *scl;  // this lane's 16 scale bytes of block `wave` of chunk 0
@@ -786,15 +800,15 @@ struct Tiles256 {
     const int tid = threadIdx.x;
     wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     lane = tid & 63;
-    wm = wave & 3;
-    wn = wave >> 2;
+    wm = wave % W::kWaveRows;
+    wn = wave / W::kWaveRows;
     li = lane & 31;
     h = lane >> 5;
-    const unsigned tiles_m = static_cast<unsigned>((nr + kEBM - 1) / kEBM);
+    const unsigned tiles_m = static_cast<unsigned>((nr + kBM - 1) / kBM);
     const unsigned tiles_n = static_cast<unsigned>((nc + kEBN - 1) / kEBN);
     unsigned tm, tn;
     tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
-    m0 = static_cast<size_t>(tm) * kEBM;
+    m0 = static_cast<size_t>(tm) * kBM;
     n0 = static_cast<size_t>(tn) * kEBN;
     const size_t ngx = (nr + kTG - 1) / kTG, ngy = (nc + kTG - 1) / kTG;
     const size_t gx0 = m0 / kTG, gy0 = n0 / kTG;
@@ -822,7 +836,7 @@ struct Tiles256 {
   template <bool kAsm = false>
   __device__ int slot(int k, size_t c, int nbc, int st) const {
     if (k < kEQuantSlots) {
-      if ((k >> 1) >= nbc)
+      if ((k >> 1) >= nbc || (kBM < kEBM && wave >= kBM / kTG && wave < 4))
         return 0;
       lds_void *to = (lds_void *)(qs + st * kEStage + (k >> 1) * kEBlock + (k & 1) * kEHalf +
                                   wave * kTG * 16);
@@ -864,46 +878,50 @@ struct Tiles256 {
 
   // this lane's operands in stage 0, block 0, tile 0 (lanes 32-63: half 1 of the
   // quants; for the Q8_0 fold the zero scale rows)
-  __device__ const int8_t *qa() const { return qs + (h * kERows + wm * 64 + li) * 16; }
-  __device__ const int8_t *qb() const { return qs + (h * kERows + kEBM + wn * 128 + li) * 16; }
-  __device__ const uint16_t *hx() const { return dsh + (h ? kERows + li : wm * 64 + li); }
-  __device__ const uint16_t *hy() const { return dsh + (h ? kERows + li : kEBM + wn * 128 + li); }
+  __device__ const int8_t *qa() const { return qs + (h * kERows + wm * kRows + li) * 16; }
+  __device__ const int8_t *qb() const { return qs + (h * kERows + kEBM + wn * kToks + li) * 16; }
+  __device__ const uint16_t *hx() const { return dsh + (h ? kERows + li : wm * kRows + li); }
+  __device__ const uint16_t *hy() const { return dsh + (h ? kERows + li : kEBM + wn * kToks + li); }
   // the Q4_0 fold: d_x of the lane's weight row li, fp32 d_y of its tokens 4h..
-  __device__ const uint16_t *q4x() const { return dsh + wm * 64 + li; }
-  __device__ const float *q4y() const { return fyd + wn * 128 + 4 * h; }
+  __device__ const uint16_t *q4x() const { return dsh + wm * kRows + li; }
+  __device__ const float *q4y() const { return fyd + wn * kToks + 4 * h; }
 };
 
 // Full chunk c of the 256 x 256 kernel in stage st: the fold (`fold(after_step)`,
 // slot k of chunk c + 1 issued after its step 3k), then the wait for chunk c + 1,
 // `publish(c + 1, stage)` and the barrier.  Returns the stage of chunk c + 1.
-template <bool kAsm = false, typename Fold, typename Publish>
-__device__ __forceinline__ int chunk256(const Tiles256 &t, size_t c, int st, Fold &&fold,
+template <bool kAsm = false, typename W, typename Fold, typename Publish>
+__device__ __forceinline__ int chunk256(const Tiles256<W> &t, size_t c, int st, Fold &&fold,
                                         Publish &&publish) {
   const bool ahead = c + 1 < t.nchunks;
   const int nba = ahead ? t.blocks_of(c + 1) : 0;
   const int sta = st ^ 1;
   fold([&](int s) {
-    if (s % 3 == 0 && s / 3 <= kEQuantSlots && ahead)
-      t.template slot<kAsm>(s / 3, c + 1, nba, sta);
+    // one slot per three steps of the 2 x 4 tiles' 32, per two of the 3 x 2 tiles' 24
+    constexpr int kEvery = W::kNI * W::kNJ * kEKB > 3 * kEQuantSlots ? 3 : 2;
+    if (s % kEvery == 0 && s / kEvery <= kEQuantSlots && ahead)
+      t.template slot<kAsm>(s / kEvery, c + 1, nba, sta);
   });
   wait_dma_barrier(0, [&] { publish(c + 1, sta); });  // no wave reads stage st any more
   return sta;
 }
 
-template <bool kQ4>
+template <bool kQ4, typename W>
 __device__ __forceinline__ void gemm_tiles256_body(size_t nb, float *s, const uint8_t *tx,
                                                    const uint8_t *ty, size_t nr, size_t nc,
                                                    size_t bs, int8_t *qs, uint16_t *dsh,
                                                    float *fyd) {
-  const Tiles256 t(nb, tx, ty, nr, nc, qs, dsh, fyd);
+  const Tiles256<W> t(nb, tx, ty, nr, nc, qs, dsh, fyd);
+  constexpr int kNI = W::kNI, kNJ = W::kNJ;
+  constexpr int kRows = Tiles256<W>::kRows, kToks = Tiles256<W>::kToks;
   const int tid = threadIdx.x, li = t.li, h = t.h, wm = t.wm, wn = t.wn;
   constexpr int kHStage = kEKB * kEHRow;
 
-  float acc[2][4][16];
+  float acc[kNI][kNJ][16];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < kNI; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < kNJ; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e)
         acc[i][j][e] = 0.0f;
@@ -936,12 +954,12 @@ __device__ __forceinline__ void gemm_tiles256_body(size_t nb, float *s, const ui
     // the compiler makes every LDS read of the fast loop that follows a DMA
     // issue wait for that DMA (4096^3 185 against 155 us).
     for (; c < nfull; ++c) {
-      if (q4_chunk_nonfinite<kEHRow>(dsh + st * kHStage + wm * 64, kEKB, t.lane))
+      if (q4_chunk_nonfinite<kEHRow, kRows>(dsh + st * kHStage + wm * kRows, kEKB, t.lane))
         break;
       st = chunk256(
           t, c, st,
           [&](auto after_step) {
-            fold_chunk_q4_2x4<false, kEKB, kEBlock, 32 * 16, kEHRow, kEBN>(
+            fold_chunk_q4_tiles<false, kNI, kNJ, kEKB, kEBlock, 32 * 16, kEHRow, kEBN>(
                 acc, qa + st * kEStage, qb + st * kEStage, qx + st * kHStage,
                 qy + st * kEFyStage, after_step);
           },
@@ -951,13 +969,13 @@ __device__ __forceinline__ void gemm_tiles256_body(size_t nb, float *s, const ui
       st = chunk256<true>(
           t, c, st,
           [&](auto after_step) {
-            fold_chunk_q4_2x4<true, kEKB, kEBlock, 32 * 16, kEHRow, kEBN>(
+            fold_chunk_q4_tiles<true, kNI, kNJ, kEKB, kEBlock, 32 * 16, kEHRow, kEBN>(
                 acc, qa + st * kEStage, qb + st * kEStage, qx + st * kHStage,
                 qy + st * kEFyStage, after_step);
           },
           publish);
     if (nbc > 0)
-      fold_tail_q4_2x4<true, kEBlock, 32 * 16, kEHRow, kEBN>(
+      fold_tail_q4_tiles<true, kNI, kNJ, kEBlock, 32 * 16, kEHRow, kEBN>(
           acc, qa + st * kEStage, qb + st * kEStage, qx + st * kHStage, qy + st * kEFyStage, nbc);
     // Lane (li, h) holds weight row li of tile (i, j) and its tokens 8g + 4h + e:
     // each tile goes through a wave-private 32 x 33 fp32 buffer in the quant
@@ -967,18 +985,18 @@ __device__ __forceinline__ void gemm_tiles256_body(size_t nb, float *s, const ui
     float *tb =
         reinterpret_cast<float *>(qs + (nbc > 0 ? 1 - st : st) * kEStage) + t.wave * 32 * 33;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < kNI; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < kNJ; ++j) {
 #pragma unroll
         for (int e = 0; e < 16; ++e)
           tb[li * 33 + 8 * (e >> 2) + 4 * h + (e & 3)] = acc[i][j][e];
         __builtin_amdgcn_wave_barrier();
-        const size_t col = n0 + wn * 128 + j * 32 + li;
+        const size_t col = n0 + wn * kToks + j * 32 + li;
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
           const int r = 2 * k + h;  // this half-wave's weight row of the tile
-          const size_t row = m0 + wm * 64 + i * 32 + r;
+          const size_t row = m0 + wm * kRows + i * 32 + r;
           const float v = tb[r * 33 + li];
           if (row < nr && col < nc)
             s[row * bs + col] = v;
@@ -991,22 +1009,22 @@ __device__ __forceinline__ void gemm_tiles256_body(size_t nb, float *s, const ui
       st = chunk256(
           t, c, st,
           [&](auto after_step) {
-            fold_chunk_q8_2x4<kEKB, kEBlock, 32 * 16, kEHRow>(
+            fold_chunk_q8_tiles<kNI, kNJ, kEKB, kEBlock, 32 * 16, kEHRow>(
                 acc, qa + st * kEStage, qb + st * kEStage, hx + st * kHStage, hy + st * kHStage,
                 after_step);
           },
           publish);
     if (nbc > 0)
-      fold_tail_q8_2x4<kEBlock, 32 * 16, kEHRow>(acc, qa + st * kEStage, qb + st * kEStage,
+      fold_tail_q8_tiles<kNI, kNJ, kEBlock, 32 * 16, kEHRow>(acc, qa + st * kEStage, qb + st * kEStage,
                                                  hx + st * kHStage, hy + st * kHStage, nbc);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const size_t col = n0 + wn * 128 + j * 32 + li;
+    for (int j = 0; j < kNJ; ++j) {
+      const size_t col = n0 + wn * kToks + j * 32 + li;
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < kNI; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          const size_t row = m0 + wm * 64 + i * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
+          const size_t row = m0 + wm * kRows + i * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
           if (row < nr && col < nc)
             s[row * bs + col] = acc[i][j][e];
         }
@@ -1014,15 +1032,17 @@ __device__ __forceinline__ void gemm_tiles256_body(size_t nb, float *s, const ui
   }
 }
 
+template <typename W>
 __global__ __launch_bounds__(kEThreads, 1) void gemm_tiles256_q8(size_t nb, float *s,
                                                                  const uint8_t *tx,
                                                                  const uint8_t *ty, size_t nr,
                                                                  size_t nc, size_t bs) {
   __shared__ __align__(16) int8_t qs[kEStages * kEStage];
   __shared__ __align__(16) uint16_t dsh[kEStages * kEKB * kEHRow];
-  gemm_tiles256_body<false>(nb, s, tx, ty, nr, nc, bs, qs, dsh, nullptr);
+  gemm_tiles256_body<false, W>(nb, s, tx, ty, nr, nc, bs, qs, dsh, nullptr);
 }
 
+template <typename W>
 __global__ __launch_bounds__(kEThreads, 1) void gemm_tiles256_q4(size_t nb, float *s,
                                                                  const uint8_t *tx,
                                                                  const uint8_t *ty, size_t nr,
@@ -1030,7 +1050,7 @@ __global__ __launch_bounds__(kEThreads, 1) void gemm_tiles256_q4(size_t nb, floa
   __shared__ __align__(16) int8_t qs[kEStages * kEStage];
   __shared__ __align__(16) uint16_t dsh[kEStages * kEKB * kEHRow];
   __shared__ __align__(16) float fyd[kEStages * kEFyStage];
-  gemm_tiles256_body<true>(nb, s, tx, ty, nr, nc, bs, qs, dsh, fyd);
+  gemm_tiles256_body<true, W>(nb, s, tx, ty, nr, nc, bs, qs, dsh, fyd);
 }
 
 // ---- few work-group tiles: one 32 x 32 tile a wave, no LDS -----------------
@@ -1650,29 +1670,38 @@ int pack_tiles_both(size_t nb, const uint8_t *vx, size_t bx, size_t nr, uint8_t 
   return launch_status();
 }
 
-// Which Q8_0 kernel serves a shape: both fold every output in the same order, so
-// the choice is speed only.  One MI355X runs 256 work-groups of either kernel at
-// once (one per CU); a round of 256 x 256 tiles takes ~1.87 times a round of
-// 256 x 128 ones at equal K (4096^3: one round 150-152 us against two rounds in
-// 161 us), and a lone round of the smaller tile 93 us.  So the larger tile runs
-// when its rounds x 15 are at most the smaller tile's rounds x 8: at 4096 x 4096
-// outputs (one round against two) and at 8192 x 4096 (two against four), not at
-// 4096 x 2048 (half the CUs idle) or 4196 x 4166 (two against three).
-bool tiles256_first(size_t tiles, size_t tiles256) {
+// Which work-group tile serves a shape: all fold every output in the same order, so
+// the choice is speed only.  One MI355X runs 256 work-groups of any of them at
+// once (one per CU).  A round takes (us, K 4096, Q4_0 / Q8_0) 155-165 / 139-148
+// of 256 x 256 tiles, 127-133 / 108-119 of 192 x 256, 90-99 / 75-89 of 256 x 128: the
+// fewest rounds x 32, 26 and 18.  Measured, 256 / 192 / 128: 4096 x 4096 165 / 250 / 182,
+// 148 / 215 / 161; 11008 x 1000 155 / 129 / 181, 139 / 119 / 153; 4196 x 4166 304 / 250 /
+// 270, 275 / 217 / 229; 14336 x 700 155 / 128 / 176, 142 / 115 / 148; 4096 x 2048 155 / 127
+// / 99, 137 / 109 / 87; 6000 x 2500 165 / 250 / 186, 153 / 214 / 159.
+enum class TileShape { k256x256, k192x256, k256x128 };
+TileShape tile_shape(size_t tiles256, size_t tiles192, size_t tiles128) {
   constexpr size_t kCUs = 256;
-  return (tiles256 + kCUs - 1) / kCUs * 15 <= (tiles + kCUs - 1) / kCUs * 8;
+  const size_t c256 = (tiles256 + kCUs - 1) / kCUs * 32, c192 = (tiles192 + kCUs - 1) / kCUs * 26,
+               c128 = (tiles128 + kCUs - 1) / kCUs * 18;
+  if (c256 <= c192 && c256 <= c128)
+    return TileShape::k256x256;
+  return c192 <= c128 ? TileShape::k192x256 : TileShape::k256x128;
 }
 
 // Few work-group tiles: the one-tile-a-wave kernel where the 256 x 128 tiles
-// would not fill one round of the CUs and its own waves fit two rounds of two
-// a SIMD (at most 1024 work-groups).  Pre-packed operands, K 4096 unless
-// named, us, 256 x 128 tiles against it: 4096 x 128 72 / 17, 4096 x 512 74 /
-// 28, 4096 x 1024 75 / 53, 14336 x 128 72 / 27, 4096 x 128 x 14336 234 / 51;
-// but 14336 x 512 (1792 of its work-groups) 82 / 88, and from 256 tiles (a
+// would not fill one round of the CUs and its own work-groups are few.  Pre-packed
+// operands, K 4096 unless named, us, 256 x 128 tiles against it: 4096 x 128 72 / 17, 4096 x
+// 512 74 / 28, 4096 x 1024 75 / 53, 14336 x 128 72 / 27, 4096 x 128 x 14336 234 / 51;
+// 14336 x 300 (1120 of its work-groups) 90 / 70 Q4_0, 75 / 61 Q8_0, 2048 x 3000 (1504)
+// 92 / 84, 78 / 77; but 4096 x 1700 (1728) 93 / 95, 79 / 86, and from 256 tiles (a
 // full round) the larger tiles win: 4096 x 2048 93-98 against ~100.
-bool tiles32_first(size_t tiles, size_t tiles64, size_t nb) {
-  return tiles < 256 && tiles64 <= 1024 && nb <= 0xffffffffu;
+constexpr size_t kTiles32Max = 1536;
+bool tiles32_first(size_t tiles, size_t tiles64, size_t nb, size_t most = kTiles32Max) {
+  return tiles < 256 && tiles64 <= most && nb <= 0xffffffffu;
 }
+// From plain rows (gemm_rows_few) at 1024 the 256-row kernels are as fast: 4096 x 1024 x
+// 4096 Q8_0 91.6 against 91-93 us.
+constexpr size_t kRowsFewMax = 1024;
 
 // Fewer still: one 16 x 16 tile a wave while its waves fit one a SIMD (at most
 // 256 work-groups of 32 x 32).  Pre-packed, K 4096, us, 32 x 32 tiles against
@@ -1695,8 +1724,8 @@ int gemm_tiles(size_t nb, float *s, const uint8_t *tx, const uint8_t *ty, size_t
   const size_t tiles = ((nr + tcrv::kDBM - 1) / tcrv::kDBM) * ((nc + tcrv::kDBN - 1) / tcrv::kDBN);
   if (tiles > 0x7fffffffu)
     return TCRV_HIP_ERR_TOO_LARGE;
-  const size_t tiles256 =
-      ((nr + tcrv::kEBM - 1) / tcrv::kEBM) * ((nc + tcrv::kEBN - 1) / tcrv::kEBN);
+  const size_t tn256 = (nc + tcrv::kEBN - 1) / tcrv::kEBN;
+  const size_t tiles256 = ((nr + 255) / 256) * tn256, tiles192 = ((nr + 191) / 192) * tn256;
   const size_t tiles64 =
       ((nr + tcrv::kSBM - 1) / tcrv::kSBM) * ((nc + tcrv::kSBN - 1) / tcrv::kSBN);
   if (tiles32_first(tiles, tiles64, nb) && tiles16_first(nr, nc)) {
@@ -1717,18 +1746,25 @@ int gemm_tiles(size_t nb, float *s, const uint8_t *tx, const uint8_t *ty, size_t
     else
       tcrv::gemm_tiles32<false><<<dim3(static_cast<unsigned>(tiles64)), dim3(256), 0, st>>>(
           nbu, s, tx, ty, nr, nc, bs);
-  } else if (q4 && nb <= kMaxTiledNb && tiles256_first(tiles, tiles256))
-    tcrv::gemm_tiles256_q4<<<dim3(static_cast<unsigned>(tiles256)), dim3(tcrv::kEThreads), 0,
-                             st>>>(nb, s, tx, ty, nr, nc, bs);
-  else if (q4)
-    tcrv::gemm_tiles_q4<<<dim3(static_cast<unsigned>(tiles)), dim3(tcrv::kDThreads), 0, st>>>(
-        nb, s, tx, ty, nr, nc, bs);
-  else if (tiles256_first(tiles, tiles256))
-    tcrv::gemm_tiles256_q8<<<dim3(static_cast<unsigned>(tiles256)), dim3(tcrv::kEThreads), 0,
-                             st>>>(nb, s, tx, ty, nr, nc, bs);
-  else
-    tcrv::gemm_tiles_q8<kTiledPipe><<<dim3(static_cast<unsigned>(tiles)),
-                                      dim3(tcrv::kDThreads), 0, st>>>(nb, s, tx, ty, nr, nc, bs);
+  } else {
+    const TileShape shape = q4 && nb > kMaxTiledNb ? TileShape::k256x128
+                                                   : tile_shape(tiles256, tiles192, tiles);
+    const size_t n = shape == TileShape::k256x256   ? tiles256
+                     : shape == TileShape::k192x256 ? tiles192
+                                                    : tiles;
+    auto run = [&](auto kernel, int threads) {
+      kernel<<<dim3(static_cast<unsigned>(n)), dim3(threads), 0, st>>>(nb, s, tx, ty, nr, nc, bs);
+    };
+    if (shape == TileShape::k256x256)
+      q4 ? run(tcrv::gemm_tiles256_q4<tcrv::Wave2x4>, tcrv::kEThreads)
+         : run(tcrv::gemm_tiles256_q8<tcrv::Wave2x4>, tcrv::kEThreads);
+    else if (shape == TileShape::k192x256)
+      q4 ? run(tcrv::gemm_tiles256_q4<tcrv::Wave3x2>, tcrv::kEThreads)
+         : run(tcrv::gemm_tiles256_q8<tcrv::Wave3x2>, tcrv::kEThreads);
+    else
+      q4 ? run(tcrv::gemm_tiles_q4, tcrv::kDThreads)
+         : run(tcrv::gemm_tiles_q8<kTiledPipe>, tcrv::kDThreads);
+  }
   return launch_status();
 }
 
@@ -1777,13 +1813,12 @@ namespace tcrv_host {
 
 // The plain-row entries' kernel for shapes of few output tiles (gemm_rows_few):
 // rows 16-byte aligned, a whole number of 8-block chunks, the shapes
-// gemm_tiles32 serves (at its 1024 work-groups the 256-row kernels are as fast:
-// 4096 x 1024 x 4096 Q8_0 91.6 against 91-93 us).
+// gemm_tiles32 serves up to kRowsFewMax work-groups.
 bool rows_few_serves(size_t nb, const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by,
                      size_t nr, size_t nc) {
   return nr >= 2 && nc >= 2 && nb != 0 && nb % tcrv::kFKB == 0 && aligned16(vx) &&
          aligned16(vy) && bx % 16 == 0 && by % 16 == 0 &&
-         tiles32_first(tiles128_of(nr, nc), tiles64_of(nr, nc), nb);
+         tiles32_first(tiles128_of(nr, nc), tiles64_of(nr, nc), nb, kRowsFewMax);
 }
 
 int gemm_rows_few(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
@@ -1960,3 +1995,4 @@ int tcrv_hip_q4_0_q8_0_gemm_ws(size_t n, float *s, const uint8_t *vx, const uint
 }
 
 }  // extern "C"
+

@@ -198,36 +198,40 @@ __device__ __forceinline__ void fold_tail_q8(float (&acc)[2][16], const int8_t *
   }
 }
 
-// ---- the Q8_0 fold over 2 x 4 tiles per wave ------------------------------
-// One chunk of kBlocks blocks for a wave's two weight tiles (A operand at
-// qa + i * kTile bytes, d_x at hx + 32 i) and four token tiles (B operand at
+// ---- the Q8_0 fold over kNI x kNJ tiles per wave (2 x 4 or 3 x 2) -----------
+// One chunk of kBlocks blocks for a wave's kNI weight tiles (A operand at
+// qa + i * kTile bytes, d_x at hx + 32 i) and kNJ token tiles (B operand at
 // qb + j * kTile, d_y at hy + 32 j); block b is kBlockStride bytes and
-// kScaleRow scales further.  Steps s = 8b + 2j + i, so every tile's blocks are
+// kScaleRow scales further.  Steps s = (b, j, i), i fastest, so every tile's blocks are
 // folded in ascending order.  As in fold_chunk_q8 the block-sum MFMA of step
 // s+1 is issued in step s; here every LDS read also lands a whole step before
 // the MFMA that takes it (two waves per SIMD hide less latency than four): the
 // token operand and d_y of tile j+1 are read in step (b, j, 0), the next
-// block's weight operands and d_x in steps (b, 3, 0), (b, 3, 1) and
-// (b+1, 0, 0), each into the registers of an operand whose last MFMA has been
-// issued (two weight and two token fragments, two d_x and two d_y words).
-template <int kBlocks, int kBlockStride, int kTile, int kScaleRow, typename AfterStep>
-__device__ __forceinline__ void fold_chunk_q8_2x4(float (&acc)[2][4][16], const int8_t *qa,
-                                                  const int8_t *qb, const uint16_t *hx,
-                                                  const uint16_t *hy, AfterStep &&after_step) {
-  v4i w[2], t[2];
-  uint32_t ux[2], uy[2];
-  w[0] = q8_frag<kBlockStride>(qa, 0);
-  w[1] = q8_frag<kBlockStride>(qa + kTile, 0);
+// block's weight operand i in step (b, kNJ-1, i) and its d_x in the step after,
+// each into the registers of an operand whose last MFMA has been
+// issued (kNI weight and two token fragments, kNI d_x and two d_y words).
+template <int kNI, int kNJ, int kBlocks, int kBlockStride, int kTile, int kScaleRow,
+          typename AfterStep>
+__device__ __forceinline__ void fold_chunk_q8_tiles(float (&acc)[kNI][kNJ][16], const int8_t *qa,
+                                                    const int8_t *qb, const uint16_t *hx,
+                                                    const uint16_t *hy, AfterStep &&after_step) {
+  static_assert(kNJ % 2 == 0, "token operands alternate between two register sets");
+  constexpr int kSteps = kNI * kNJ;
+  v4i w[kNI], t[2];
+  uint32_t ux[kNI], uy[2];
+#pragma unroll
+  for (int i = 0; i < kNI; ++i) {
+    w[i] = q8_frag<kBlockStride>(qa + i * kTile, 0);
+    ux[i] = q8_scale<kScaleRow>(hx + 32 * i, 0);
+  }
   t[0] = q8_frag<kBlockStride>(qb, 0);
-  ux[0] = q8_scale<kScaleRow>(hx, 0);
-  ux[1] = q8_scale<kScaleRow>(hx + 32, 0);
   uy[0] = q8_scale<kScaleRow>(hy, 0);
   v16i cur = q8_sumi(w[0], t[0]);
 #pragma unroll
-  for (int s = 0; s < 8 * kBlocks; ++s) {
-    const int b = s >> 3, j = (s >> 1) & 3, i = s & 1;
+  for (int s = 0; s < kSteps * kBlocks; ++s) {
+    const int b = s / kSteps, j = s % kSteps / kNI, i = s % kNI;
     if (i == 0) {
-      if (j < 3) {
+      if (j < kNJ - 1) {
         t[(j + 1) & 1] = q8_frag<kBlockStride>(qb + (j + 1) * kTile, b);
         uy[(j + 1) & 1] = q8_scale<kScaleRow>(hy + 32 * (j + 1), b);
       } else if (b + 1 < kBlocks) {
@@ -236,17 +240,17 @@ __device__ __forceinline__ void fold_chunk_q8_2x4(float (&acc)[2][4][16], const 
         w[0] = q8_frag<kBlockStride>(qa, b + 1);
       }
       if (j == 0 && b > 0)
-        ux[1] = q8_scale<kScaleRow>(hx + 32, b);
-    } else if (j == 3 && b + 1 < kBlocks) {
-      w[1] = q8_frag<kBlockStride>(qa + kTile, b + 1);
-      ux[0] = q8_scale<kScaleRow>(hx, b + 1);
+        ux[kNI - 1] = q8_scale<kScaleRow>(hx + 32 * (kNI - 1), b);
+    } else if (j == kNJ - 1 && b + 1 < kBlocks) {
+      w[i] = q8_frag<kBlockStride>(qa + i * kTile, b + 1);
+      ux[i - 1] = q8_scale<kScaleRow>(hx + 32 * (i - 1), b + 1);
     }
     v16i nxt;
-    if (s + 1 < 8 * kBlocks)
-      nxt = q8_sumi(w[(s + 1) & 1], t[((s + 1) >> 1) & 1]);
+    if (s + 1 < kSteps * kBlocks)
+      nxt = q8_sumi(w[(s + 1) % kNI], t[(s + 1) / kNI & 1]);
     const v16f dxy = q8_dxy(ux[i], uy[j & 1]);
     q8_fold<true>(acc[i][j], cur, dxy);
-    if (s + 1 < 8 * kBlocks) {
+    if (s + 1 < kSteps * kBlocks) {
       asm volatile("" : "+v"(nxt));
       cur = nxt;
     }
@@ -258,20 +262,26 @@ __device__ __forceinline__ void fold_chunk_q8_2x4(float (&acc)[2][4][16], const 
   }
 }
 
-// A trailing partial chunk of nbc blocks over the 2 x 4 tiles, one step at a time.
-template <int kBlockStride, int kTile, int kScaleRow>
-__device__ __forceinline__ void fold_tail_q8_2x4(float (&acc)[2][4][16], const int8_t *qa,
-                                                 const int8_t *qb, const uint16_t *hx,
-                                                 const uint16_t *hy, int nbc) {
+// A trailing partial chunk of nbc blocks over the tiles, one step at a time.
+template <int kNI, int kNJ, int kBlockStride, int kTile, int kScaleRow>
+__device__ __forceinline__ void fold_tail_q8_tiles(float (&acc)[kNI][kNJ][16], const int8_t *qa,
+                                                   const int8_t *qb, const uint16_t *hx,
+                                                   const uint16_t *hy, int nbc) {
   for (int b = 0; b < nbc; ++b) {
-    const v4i w0 = q8_frag<kBlockStride>(qa, b), w1 = q8_frag<kBlockStride>(qa + kTile, b);
-    const uint32_t ux0 = q8_scale<kScaleRow>(hx, b), ux1 = q8_scale<kScaleRow>(hx + 32, b);
+    v4i w[kNI];
+    uint32_t ux[kNI];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int i = 0; i < kNI; ++i) {
+      w[i] = q8_frag<kBlockStride>(qa + i * kTile, b);
+      ux[i] = q8_scale<kScaleRow>(hx + 32 * i, b);
+    }
+#pragma unroll
+    for (int j = 0; j < kNJ; ++j) {
       const v4i t = q8_frag<kBlockStride>(qb + j * kTile, b);
       const uint32_t uy = q8_scale<kScaleRow>(hy + 32 * j, b);
-      q8_fold(acc[0][j], q8_sumi(w0, t), q8_dxy(ux0, uy));
-      q8_fold(acc[1][j], q8_sumi(w1, t), q8_dxy(ux1, uy));
+#pragma unroll
+      for (int i = 0; i < kNI; ++i)
+        q8_fold(acc[i][j], q8_sumi(w[i], t), q8_dxy(ux[i], uy));
     }
   }
 }
@@ -323,14 +333,14 @@ __device__ __forceinline__ float f16_bits(uint32_t u) {
   return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(u)));
 }
 
-// Whether any d_x of the wave's 64 weight rows in the chunk's nbc blocks is
-// non-finite (exponent field all ones; NaN is included, which only costs the
-// exact form): lane 8b + k reads rows 8k..8k+7 of block b as one 128-bit LDS
+// Whether any d_x of the wave's kRows weight rows in the chunk's nbc blocks (at most 512 /
+// kRows) is non-finite (exponent field all ones; NaN is included, which only costs the
+// exact form): lane (kRows / 8) b + k reads rows 8k..8k+7 of block b as one 128-bit LDS
 // read, and (h & 0x7C00) + 0x0400 reaches bit 15 exactly when h's exponent is
 // 0x1F (no carry crosses into the other half).  hx: the wave's row 0, block 0.
-template <int kScaleRow>
+template <int kScaleRow, int kRows = 64>
 __device__ __forceinline__ bool q4_chunk_nonfinite(const uint16_t *hx, int nbc, int lane) {
-  const int b = lane >> 3, k = lane & 7;
+  const int b = lane / (kRows / 8), k = lane % (kRows / 8);
   uint32_t top = 0;
   if (b < nbc) {
     const uint4 w = *reinterpret_cast<const uint4 *>(hx + b * kScaleRow + 8 * k);
@@ -421,7 +431,7 @@ __device__ __forceinline__ void fold_tail_q4(float (&acc)[2][16], const int8_t *
   }
 }
 
-// ---- the Q4_0 fold over 2 x 4 tiles per wave ------------------------------
+// ---- the Q4_0 fold over 2 x 4 or 3 x 2 tiles per wave ---------------------
 // The fold of one tile and block with d_y already in registers (dy[e]: the
 // token of accumulator element e); every fl(sumi * d_x) of the step is formed
 // before the first fma that takes one, so the d_y reads issued at the step's
@@ -460,28 +470,29 @@ __device__ __forceinline__ void q4_read_dy(float (&dy)[16], const float *fy) {
   }
 }
 
-// One chunk of kBlocks blocks for a wave's two weight tiles (B operand at
-// qw + i * kTile, d_x at hx + 32 i) and four token tiles (A operand at
+// One chunk of kBlocks blocks for a wave's kNI weight tiles (B operand at
+// qw + i * kTile, d_x at hx + 32 i) and kNJ token tiles (A operand at
 // qt + j * kTile, fp32 d_y at fy + 32 j, block b kFyRow floats on) on
-// transposed 32 x 32 tiles, steps s = 8b + 2j + i: every tile's blocks in
+// transposed 32 x 32 tiles, steps s = (b, j, i), i fastest: every tile's blocks in
 // ascending order.  The seeded MFMA of step s+1 is issued in step s; the
-// operand reads follow fold_chunk_q8_2x4's schedule (token tile j+1 in step
-// (b, j, 0), the next block's weight operands in steps (b, 3, 0) and
-// (b, 3, 1)); a token tile's d_y is read once per block, in its step i = 0,
-// and serves both weight tiles.
-template <bool kExact, int kBlocks, int kBlockStride, int kTile, int kScaleRow, int kFyRow,
-          typename AfterStep>
-__device__ __forceinline__ void fold_chunk_q4_2x4(float (&acc)[2][4][16], const int8_t *qw,
-                                                  const int8_t *qt, const uint16_t *hx,
-                                                  const float *fy, AfterStep &&after_step) {
-  v4i w[2], t[2];
-  uint32_t ux[2];
+// operand reads follow fold_chunk_q8_tiles's schedule; a token tile's d_y is read once per
+// block, in its step i = 0, and serves every weight tile.
+template <bool kExact, int kNI, int kNJ, int kBlocks, int kBlockStride, int kTile, int kScaleRow,
+          int kFyRow, typename AfterStep>
+__device__ __forceinline__ void fold_chunk_q4_tiles(float (&acc)[kNI][kNJ][16], const int8_t *qw,
+                                                    const int8_t *qt, const uint16_t *hx,
+                                                    const float *fy, AfterStep &&after_step) {
+  static_assert(kNJ % 2 == 0, "token operands alternate between two register sets");
+  constexpr int kSteps = kNI * kNJ;
+  v4i w[kNI], t[2];
+  uint32_t ux[kNI];
   float dy[16];
-  w[0] = q8_frag<kBlockStride>(qw, 0);
-  w[1] = q8_frag<kBlockStride>(qw + kTile, 0);
+#pragma unroll
+  for (int i = 0; i < kNI; ++i) {
+    w[i] = q8_frag<kBlockStride>(qw + i * kTile, 0);
+    ux[i] = q8_scale<kScaleRow>(hx + 32 * i, 0);
+  }
   t[0] = q8_frag<kBlockStride>(qt, 0);
-  ux[0] = q8_scale<kScaleRow>(hx, 0);
-  ux[1] = q8_scale<kScaleRow>(hx + 32, 0);
   // the seed, hidden from instruction selection: as a known constant it is
   // rebuilt from scalar registers (24 instructions) each time register
   // pressure evicts it
@@ -495,26 +506,26 @@ __device__ __forceinline__ void fold_chunk_q4_2x4(float (&acc)[2][4][16], const 
   };
   v16f cur = sums(t[0], w[0]);
 #pragma unroll
-  for (int s = 0; s < 8 * kBlocks; ++s) {
-    const int b = s >> 3, j = (s >> 1) & 3, i = s & 1;
+  for (int s = 0; s < kSteps * kBlocks; ++s) {
+    const int b = s / kSteps, j = s % kSteps / kNI, i = s % kNI;
     if (i == 0) {
       q4_read_dy(dy, fy + b * kFyRow + 32 * j);
-      if (j < 3) {
+      if (j < kNJ - 1) {
         t[(j + 1) & 1] = q8_frag<kBlockStride>(qt + (j + 1) * kTile, b);
       } else if (b + 1 < kBlocks) {
         t[0] = q8_frag<kBlockStride>(qt, b + 1);
         w[0] = q8_frag<kBlockStride>(qw, b + 1);
       }
-    } else if (j == 3 && b + 1 < kBlocks) {
-      w[1] = q8_frag<kBlockStride>(qw + kTile, b + 1);
+    } else if (j == kNJ - 1 && b + 1 < kBlocks) {
+      w[i] = q8_frag<kBlockStride>(qw + i * kTile, b + 1);
     }
     v16f nxt;
-    if (s + 1 < 8 * kBlocks)
-      nxt = sums(t[((s + 1) >> 1) & 1], w[(s + 1) & 1]);
+    if (s + 1 < kSteps * kBlocks)
+      nxt = sums(t[(s + 1) / kNI & 1], w[(s + 1) % kNI]);
     q4_fold_dy<kExact>(acc[i][j], cur, ux[i], dy);
-    if (j == 3 && b + 1 < kBlocks)  // this block's last use of d_x of tile i
+    if (j == kNJ - 1 && b + 1 < kBlocks)  // this block's last use of d_x of tile i
       ux[i] = q8_scale<kScaleRow>(hx + 32 * i, b + 1);
-    if (s + 1 < 8 * kBlocks) {
+    if (s + 1 < kSteps * kBlocks) {
       asm volatile("" : "+v"(nxt));
       cur = nxt;
     }
@@ -523,21 +534,27 @@ __device__ __forceinline__ void fold_chunk_q4_2x4(float (&acc)[2][4][16], const 
   }
 }
 
-// A trailing partial chunk of nbc blocks over the 2 x 4 transposed tiles.
-template <bool kExact, int kBlockStride, int kTile, int kScaleRow, int kFyRow>
-__device__ __forceinline__ void fold_tail_q4_2x4(float (&acc)[2][4][16], const int8_t *qw,
-                                                 const int8_t *qt, const uint16_t *hx,
-                                                 const float *fy, int nbc) {
+// A trailing partial chunk of nbc blocks over the transposed tiles.
+template <bool kExact, int kNI, int kNJ, int kBlockStride, int kTile, int kScaleRow, int kFyRow>
+__device__ __forceinline__ void fold_tail_q4_tiles(float (&acc)[kNI][kNJ][16], const int8_t *qw,
+                                                   const int8_t *qt, const uint16_t *hx,
+                                                   const float *fy, int nbc) {
   for (int b = 0; b < nbc; ++b) {
-    const v4i w0 = q8_frag<kBlockStride>(qw, b), w1 = q8_frag<kBlockStride>(qw + kTile, b);
-    const uint32_t ux0 = q8_scale<kScaleRow>(hx, b), ux1 = q8_scale<kScaleRow>(hx + 32, b);
+    v4i w[kNI];
+    uint32_t ux[kNI];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int i = 0; i < kNI; ++i) {
+      w[i] = q8_frag<kBlockStride>(qw + i * kTile, b);
+      ux[i] = q8_scale<kScaleRow>(hx + 32 * i, b);
+    }
+#pragma unroll
+    for (int j = 0; j < kNJ; ++j) {
       const v4i tq = q8_frag<kBlockStride>(qt + j * kTile, b);
       float dy[16];
       q4_read_dy(dy, fy + b * kFyRow + 32 * j);
-      q4_fold_dy<kExact>(acc[0][j], q4_seeded_sums(tq, w0), ux0, dy);
-      q4_fold_dy<kExact>(acc[1][j], q4_seeded_sums(tq, w1), ux1, dy);
+#pragma unroll
+      for (int i = 0; i < kNI; ++i)
+        q4_fold_dy<kExact>(acc[i][j], q4_seeded_sums(tq, w[i]), ux[i], dy);
     }
   }
 }
