@@ -51,16 +51,18 @@ static_assert(kDStages * (kDKB * 12288 + kDKB * (kDBM + kDBN + 32) * 2 + kDKB * 
               "the stages fit the 160 KB of LDS");
 
 // ---------------------------------------------------------------- pack ---
-// Rows 16-byte aligned (and bx % 16 == 0): one wave per (group, 8-block range),
-// lane r = row 64g + r.  Blocks 8c..8c+7 of a row are 272 contiguous bytes at a
-// 16-byte aligned offset (8 x 34 = 17 x 16), so the lane loads them with 17
-// 128-bit loads, all issued before the first use, and the whole span of the
-// row's cache lines is read by one wave (a wave per record read each line from
-// up to three XCDs).  The eight records are then written from registers, every
-// store 64 consecutive 16-byte (or 2-byte) slots.
-constexpr int kPackSpan = 8;  // blocks per lane (4096 rows x 128 blocks: 7.3 us; the
-                              // per-record kernel 9.3 us; two waves per 8-block span
-                              // with 9 loads each 12.2 us)
+// A work-group of 4 waves per (64-row group, 8-block range), or two ranges of them.  Blocks
+// 8c..8c+7 of a row are 272 (Q4_0: 144) contiguous bytes, which the threads load in 16-byte
+// pieces, whole rows side by side (a lane per row put 64 rows' cache lines under every
+// load instruction), and put into LDS as they lie; each wave then reads its two blocks of every
+// row, lane r row r, and writes their records from registers, every store 64
+// consecutive 16-byte (or 2-byte) slots.  Rows need only 2-byte alignment (the hardware
+// takes 128-bit global loads at any), and with a block count that is no multiple of 8 the
+// last range starts at block nb - 8 and stores the blocks the one before it left.  Measured
+// (us, against a wave per range with a lane per row and, for other rows, a wave per record
+// with 16-bit loads): 4096 x 4096 Q8_0 7.0 -> 6.6; 1000 x 4096 Q8_0 4.8 ->
+// 3.4; 3001 rows of 91 blocks 6.7 -> 4.8, Q4_0 5.4 -> 4.4.
+constexpr int kPackSpan = 8;  // blocks of a range
 
 // Lane r's part of one record: its row's 32 quants (two 16-byte slots of the
 // record's 64-slot halves) and its fp16 scale.  kStream: nontemporal stores,
@@ -86,115 +88,27 @@ __device__ __forceinline__ void store_record(uint8_t *o, int r, const uint32_t (
   }
 }
 
-// Span `wave` of one operand (64-row group g, 8-block span c), lane r = row
-// 64g + r.
-template <bool kStream>
-__device__ __forceinline__ void pack_span(size_t nrows, size_t nb, const uint8_t *src,
-                                          size_t bx, uint8_t *dst, size_t wave, int r) {
-  const size_t spans_per_group = nb / kPackSpan;
-  const size_t g = wave / spans_per_group, c = wave - g * spans_per_group;
-  const size_t row = g * kTG + r;
-  uint32_t v[4 * 17];
-  if (row < nrows) {
-    const uint4 *p = reinterpret_cast<const uint4 *>(src + row * bx + c * kPackSpan * kQ8Bytes);
-#pragma unroll
-    for (int k = 0; k < 17; ++k) {
-      const uint4 x = p[k];
-      v[4 * k] = x.x; v[4 * k + 1] = x.y; v[4 * k + 2] = x.z; v[4 * k + 3] = x.w;
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < 68; ++k)
-      v[k] = 0;  // rows past nrows in the last group are zero
-  }
-#pragma unroll
-  for (int k = 0; k < kPackSpan; ++k) {
-    // block k at byte 34k of the span: even k -> dword 17k/2 holds the scale in
-    // its low half and the quants start 2 bytes in; odd k -> the scale is the
-    // high half of dword (34k-2)/4 and the quants are the next 8 dwords
-    uint32_t q[8], d;
-    if ((k & 1) == 0) {
-      const int w0 = 17 * k / 2;
-      d = v[w0] & 0xffffu;
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        q[j] = funnel16(v[w0 + j], v[w0 + j + 1]);
-    } else {
-      const int w0 = (34 * k - 2) / 4;
-      d = v[w0] >> 16;
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        q[j] = v[w0 + 1 + j];
-    }
-    store_record<kStream>(dst + (g * nb + c * kPackSpan + k) * kTRec, r, q, d);
-  }
+typedef uint32_t u32x4a2 __attribute__((ext_vector_type(4), aligned(2)));
+
+// Range `range` of an operand of nb >= 8 blocks: 64-row group g, blocks b0 .. b0 + 7, of
+// which the first `skip` belong to the range before.
+struct PackRange {
+  size_t g, b0;
+  int skip;
+};
+__device__ __forceinline__ PackRange pack_range(size_t range, size_t nb) {
+  const size_t per_group = (nb + kPackSpan - 1) / kPackSpan;
+  PackRange p;
+  p.g = range / per_group;
+  const size_t b = (range - p.g * per_group) * kPackSpan;
+  p.b0 = min(b, nb - kPackSpan);
+  p.skip = static_cast<int>(b - p.b0);
+  return p;
 }
 
-__global__ __launch_bounds__(256) void pack_gemm_tiles_span(size_t nrows, size_t nb,
-                                                            const uint8_t *src, size_t bx,
-                                                            uint8_t *dst, size_t nspans) {
-  const size_t wave = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) >> 6;
-  if (wave >= nspans)
-    return;
-  pack_span<true>(nrows, nb, src, bx, dst, wave, static_cast<int>(threadIdx.x & 63));
-}
-
-// One wave per (group, block) record for blocks b0.. of every group, lane
-// r = row 64g + r.  kAligned: the rows are 4-byte aligned (dword loads,
-// realigned with v_alignbyte for even blocks); otherwise 16-bit loads.
-template <bool kAligned>
-__global__ __launch_bounds__(256) void pack_gemm_tiles(size_t nrows, size_t nb,
-                                                       const uint8_t *src, size_t bx,
-                                                       uint8_t *dst, size_t b0, size_t nrec) {
-  const size_t t = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
-  const size_t rec = t >> 6;
-  if (rec >= nrec)
-    return;
-  const int r = static_cast<int>(t & 63);
-  const size_t per_group = nb - b0;
-  const size_t g = rec / per_group, b = b0 + (rec - g * per_group);
-  const size_t row = g * kTG + r;
-  uint32_t q[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  uint32_t d = 0;
-  if (row < nrows) {
-    const uint8_t *blk = src + row * bx + b * kQ8Bytes;
-    if constexpr (kAligned) {
-      if ((b & 1) == 0) {  // block 4-byte aligned: scale, then quants at +2
-        const uint32_t *w = reinterpret_cast<const uint32_t *>(blk);
-        uint32_t v[9];
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          v[k] = w[k];
-        v[8] = *reinterpret_cast<const uint16_t *>(blk + 32);
-        d = v[0] & 0xffffu;
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          q[k] = funnel16(v[k], v[k + 1]);
-      } else {  // quants 4-byte aligned, the scale in the dword before them
-        const uint32_t *w = reinterpret_cast<const uint32_t *>(blk - 2);
-        d = w[0] >> 16;
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          q[k] = w[k + 1];
-      }
-    } else {
-      const uint16_t *h = reinterpret_cast<const uint16_t *>(blk);
-      d = h[0];
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        q[k] = static_cast<uint32_t>(h[1 + 2 * k]) | (static_cast<uint32_t>(h[2 + 2 * k]) << 16);
-    }
-  }
-  uint8_t *o = dst + (g * nb + b) * kTRec;
-  reinterpret_cast<uint4 *>(o)[r] = make_uint4(q[0], q[1], q[2], q[3]);
-  reinterpret_cast<uint4 *>(o + 1024)[r] = make_uint4(q[4], q[5], q[6], q[7]);
-  reinterpret_cast<uint16_t *>(o + 2048)[r] = static_cast<uint16_t>(d);
-}
-
-// Q4_0 rows into the same layout with every nibble decoded to the int8 it
-// stands for (n - 8): quants 0-15 are the low nibbles of the 16 quant bytes,
-// 16-31 the high nibbles.  The subtraction is bytewise and carry-free:
-// n + 0x78 stays below 0x100, and flipping bit 7 maps it to n - 8.
+// Q4_0 nibbles decoded to the int8 they stand for (n - 8): quants 0-15 are the low
+// nibbles of the 16 quant bytes, 16-31 the high nibbles.  The subtraction is bytewise and
+// carry-free: n + 0x78 stays below 0x100, and flipping bit 7 maps it to n - 8.
 __device__ __forceinline__ void decode_q4_quants(const uint32_t w[4], uint32_t q[8]) {
 #pragma unroll
   for (int m = 0; m < 4; ++m) {
@@ -203,10 +117,120 @@ __device__ __forceinline__ void decode_q4_quants(const uint32_t w[4], uint32_t q
   }
 }
 
+// Blocks 2kPair, 2kPair + 1 of a range from its raw spans in LDS, lane r = row r: the
+// 16-byte pieces over the pair (68 or 36 bytes at 68 kPair or 36 kPair; 16 lanes at the
+// span's stride cover the 64 banks), then as the blocks lie -- the even one's scale is the
+// low half of its first dword and its quants start 2 bytes in, the odd one's scale is
+// the high half of the dword before its quants.
+template <bool kQ4, bool kStream, int kPair>
+__device__ __forceinline__ void pack_pair(const uint8_t *raw, const PackRange &pr, size_t nrows,
+                                          size_t nb, uint8_t *dst) {
+  constexpr int kBytes = kQ4 ? kQ4Bytes : kQ8Bytes, kQ = kQ4 ? 4 : 8;  // quant dwords a block
+  constexpr int kFrom = 2 * kBytes * kPair / 16, kTo = (2 * kBytes * (kPair + 1) + 15) / 16;
+  constexpr int w0 = (2 * kBytes * kPair - 16 * kFrom) / 4;  // the pair's first dword in v
+  const int r = static_cast<int>(threadIdx.x & 63);
+  const uint4 *p = reinterpret_cast<const uint4 *>(raw + r * (kPackSpan * kBytes)) + kFrom;
+  uint32_t v[4 * (kTo - kFrom)];
+#pragma unroll
+  for (int k = 0; k < kTo - kFrom; ++k) {
+    const uint4 x = p[k];
+    v[4 * k] = x.x; v[4 * k + 1] = x.y; v[4 * k + 2] = x.z; v[4 * k + 3] = x.w;
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    uint32_t w[kQ], q[8];
+    const uint32_t d = h == 0 ? v[w0] & 0xffffu : v[w0 + kQ] >> 16;
+#pragma unroll
+    for (int j = 0; j < kQ; ++j)
+      w[j] = h == 0 ? funnel16(v[w0 + j], v[w0 + j + 1]) : v[w0 + kQ + 1 + j];
+    if constexpr (kQ4) {
+      decode_q4_quants(w, q);
+      if (pr.g * kTG + r >= nrows) {  // a row past nrows: zero quants, not decoded zero nibbles
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          q[j] = 0;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        q[j] = w[j];
+    }
+    if (2 * kPair + h >= pr.skip)
+      store_record<kStream>(dst + (pr.g * nb + pr.b0 + 2 * kPair + h) * kTRec, r, q, d);
+  }
+}
+
+// Ranges kR * wg .. + kR - 1 of one operand (kQ4: Q4_0 weights) by a work-group of 4 waves.
+template <bool kQ4, bool kStream, int kR>
+__device__ __forceinline__ void pack_range_rows(size_t nrows, size_t nb, const uint8_t *src,
+                                                size_t bx, uint8_t *dst, size_t wg,
+                                                size_t nranges, uint8_t *raw) {
+  constexpr int kSpan = kPackSpan * (kQ4 ? kQ4Bytes : kQ8Bytes);  // 144 or 272
+  constexpr int kLanes = kQ4 ? 8 : 16;           // lanes a row, and one piece more a row
+  constexpr int kMain = kTG * kLanes / 256;      // 2 or 4 loads a thread
+  const int tid = threadIdx.x;
+  u32x4a2 v[kR][kMain + 1];
+  PackRange pr[kR];
+#pragma unroll
+  for (int i = 0; i < kR; ++i) {
+    pr[i] = pack_range(min(wg * kR + i, nranges - 1), nb);
+    const uint8_t *first = src + pr[i].b0 * (kQ4 ? kQ4Bytes : kQ8Bytes);
+    // rows past nrows in the last group are zero
+#pragma unroll
+    for (int j = 0; j < kMain; ++j) {
+      const size_t row = pr[i].g * kTG + j * (256 / kLanes) + tid / kLanes;
+      v[i][j] = row < nrows
+                    ? *reinterpret_cast<const u32x4a2 *>(first + row * bx + 16 * (tid % kLanes))
+                    : u32x4a2{};
+    }
+    if (tid < kTG) {
+      const size_t row = pr[i].g * kTG + tid;
+      v[i][kMain] = row < nrows
+                        ? *reinterpret_cast<const u32x4a2 *>(first + row * bx + 16 * kLanes)
+                        : u32x4a2{};
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kR; ++i) {
+    uint8_t *to = raw + i * kTG * kSpan;
+#pragma unroll
+    for (int j = 0; j < kMain; ++j)
+      *reinterpret_cast<uint4 *>(to + (j * (256 / kLanes) + tid / kLanes) * kSpan +
+                                 16 * (tid % kLanes)) =
+          make_uint4(v[i][j].x, v[i][j].y, v[i][j].z, v[i][j].w);
+    if (tid < kTG)
+      *reinterpret_cast<uint4 *>(to + tid * kSpan + 16 * kLanes) =
+          make_uint4(v[i][kMain].x, v[i][kMain].y, v[i][kMain].z, v[i][kMain].w);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kR; ++i) {
+    if (i > 0 && wg * kR + i >= nranges)
+      return;
+    const uint8_t *from = raw + i * kTG * kSpan;
+    switch (__builtin_amdgcn_readfirstlane(tid >> 6)) {
+    case 0: pack_pair<kQ4, kStream, 0>(from, pr[i], nrows, nb, dst); break;
+    case 1: pack_pair<kQ4, kStream, 1>(from, pr[i], nrows, nb, dst); break;
+    case 2: pack_pair<kQ4, kStream, 2>(from, pr[i], nrows, nb, dst); break;
+    default: pack_pair<kQ4, kStream, 3>(from, pr[i], nrows, nb, dst); break;
+    }
+  }
+}
+
+template <bool kQ4, int kR>
+__global__ __launch_bounds__(256) void pack_tiles_ranges(size_t nrows, size_t nb,
+                                                         const uint8_t *src, size_t bx,
+                                                         uint8_t *dst, size_t nranges) {
+  __shared__ __align__(16) uint8_t raw[kR * kTG * kPackSpan * (kQ4 ? kQ4Bytes : kQ8Bytes)];
+  pack_range_rows<kQ4, true, kR>(nrows, nb, src, bx, dst, blockIdx.x, nranges, raw);
+}
+
 // Span `wave` of one Q4_0 operand with 16-byte aligned rows (bx % 16 == 0):
 // 64-row group g, 8-block span c, lane r = row 64g + r; the span is 144
-// contiguous bytes (9 aligned 128-bit loads), block k at byte 18k.
-template <bool kStream>
+// contiguous bytes (9 aligned 128-bit loads), block k at byte 18k.  With waves enough that
+// their own loads cover the latency, no LDS hop and no barrier is faster, if only for 144
+// byte spans (us, against the ranges through LDS: 4096 x 4096 5.5 / 5.8, 11008 x 4096 12.5 /
+// 13.0; 1000 x 4096 3.8 / 3.1).
 __device__ __forceinline__ void pack_q4_span(size_t nrows, size_t nb, const uint8_t *src,
                                              size_t bx, uint8_t *dst, size_t wave, int r) {
   const size_t spans_per_group = nb / kPackSpan;
@@ -248,7 +272,7 @@ __device__ __forceinline__ void pack_q4_span(size_t nrows, size_t nb, const uint
       for (int j = 0; j < 8; ++j)
         q[j] = 0;  // rows past nrows in the last group are zero
     }
-    store_record<kStream>(dst + (g * nb + c * kPackSpan + k) * kTRec, r, q, d);
+    store_record<true>(dst + (g * nb + c * kPackSpan + k) * kTRec, r, q, d);
   }
 }
 
@@ -259,67 +283,73 @@ __global__ __launch_bounds__(256) void pack_q4_tiles_span(size_t nrows, size_t n
   const size_t wave = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) >> 6;
   if (wave >= nspans)
     return;
-  pack_q4_span<true>(nrows, nb, src, bx, dst, wave, static_cast<int>(threadIdx.x & 63));
+  pack_q4_span(nrows, nb, src, bx, dst, wave, static_cast<int>(threadIdx.x & 63));
 }
 
-// One wave per (group, block) record for blocks b0.. of every group (rows
-// 2-byte aligned: 16-bit loads).
-__global__ __launch_bounds__(256) void pack_q4_tiles(size_t nrows, size_t nb, const uint8_t *src,
-                                                     size_t bx, uint8_t *dst, size_t b0,
-                                                     size_t nrec) {
+// Rows of fewer than 8 blocks: one wave per (group, block) record, lane r = row 64g + r,
+// 16-bit loads.
+__global__ __launch_bounds__(256) void pack_gemm_tiles(size_t nrows, size_t nb,
+                                                       const uint8_t *src, size_t bx,
+                                                       uint8_t *dst, size_t nrec) {
   const size_t t = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
   const size_t rec = t >> 6;
   if (rec >= nrec)
     return;
   const int r = static_cast<int>(t & 63);
-  const size_t per_group = nb - b0;
-  const size_t g = rec / per_group, b = b0 + (rec - g * per_group);
+  const size_t g = rec / nb, b = rec - g * nb;
   const size_t row = g * kTG + r;
-  uint32_t w[4] = {0, 0, 0, 0}, d = 0;
+  uint32_t q[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  uint32_t d = 0;
+  if (row < nrows) {
+    const uint16_t *h = reinterpret_cast<const uint16_t *>(src + row * bx + b * kQ8Bytes);
+    d = h[0];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      q[k] = static_cast<uint32_t>(h[1 + 2 * k]) | (static_cast<uint32_t>(h[2 + 2 * k]) << 16);
+  }
+  store_record<false>(dst + rec * kTRec, r, q, d);
+}
+
+// Rows of fewer than 8 blocks: one wave per (group, block) record.
+__global__ __launch_bounds__(256) void pack_q4_tiles(size_t nrows, size_t nb, const uint8_t *src,
+                                                     size_t bx, uint8_t *dst, size_t nrec) {
+  const size_t t = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
+  const size_t rec = t >> 6;
+  if (rec >= nrec)
+    return;
+  const int r = static_cast<int>(t & 63);
+  const size_t g = rec / nb, b = rec - g * nb;
+  const size_t row = g * kTG + r;
+  uint32_t q[8] = {0, 0, 0, 0, 0, 0, 0, 0}, d = 0;
   if (row < nrows) {
     const uint16_t *hp = reinterpret_cast<const uint16_t *>(src + row * bx + b * kQ4Bytes);
+    uint32_t w[4];
     d = hp[0];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       w[j] = static_cast<uint32_t>(hp[1 + 2 * j]) | (static_cast<uint32_t>(hp[2 + 2 * j]) << 16);
+    decode_q4_quants(w, q);
   }
-  uint32_t q[8];
-  decode_q4_quants(w, q);
-  if (row >= nrows) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      q[j] = 0;
-  }
-  uint8_t *o = dst + (g * nb + b) * kTRec;
-  reinterpret_cast<uint4 *>(o)[r] = make_uint4(q[0], q[1], q[2], q[3]);
-  reinterpret_cast<uint4 *>(o + 1024)[r] = make_uint4(q[4], q[5], q[6], q[7]);
-  reinterpret_cast<uint16_t *>(o + 2048)[r] = static_cast<uint16_t>(d);
+  store_record<false>(dst + rec * kTRec, r, q, d);
 }
 
 // Both operands of one GEMM in one launch (their spans back to back in the
-// grid): one launch instead of two, and twice the loads in flight.  kXQ4: the
+// grid; nb >= 8): one launch instead of two, and twice the loads in flight.  kXQ4: the
 // first operand is Q4_0 weights.
 struct SpanOperand {
   const uint8_t *src;
-  size_t bx, nrows, nspans;
+  size_t bx, nrows, nranges;
   uint8_t *dst;
 };
 
 template <bool kXQ4>
-__global__ __launch_bounds__(256) void pack_gemm_tiles_span2(size_t nb, SpanOperand x,
-                                                             SpanOperand y) {
-  size_t wave = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) >> 6;
-  const int r = static_cast<int>(threadIdx.x & 63);
-  if (wave < x.nspans) {
-    if constexpr (kXQ4)
-      pack_q4_span<false>(x.nrows, nb, x.src, x.bx, x.dst, wave, r);
-    else
-      pack_span<false>(x.nrows, nb, x.src, x.bx, x.dst, wave, r);
-    return;
-  }
-  wave -= x.nspans;
-  if (wave < y.nspans)
-    pack_span<false>(y.nrows, nb, y.src, y.bx, y.dst, wave, r);
+__global__ __launch_bounds__(256) void pack_tiles_ranges2(size_t nb, SpanOperand x, SpanOperand y) {
+  __shared__ __align__(16) uint8_t raw[kTG * kPackSpan * kQ8Bytes];
+  if (blockIdx.x < x.nranges)
+    pack_range_rows<kXQ4, false, 1>(x.nrows, nb, x.src, x.bx, x.dst, blockIdx.x, x.nranges, raw);
+  else
+    pack_range_rows<false, false, 1>(y.nrows, nb, y.src, y.bx, y.dst, blockIdx.x - x.nranges,
+                                     y.nranges, raw);
 }
 
 // ---------------------------------------------------------------- GEMM ---
@@ -1347,7 +1377,7 @@ __global__ __launch_bounds__(256, 2) void gemm_tiles16(unsigned nb, float *s, co
 // For the reference ABI without a workspace (tcrv_hip_q8_0_q8_0_gemm,
 // tcrv_hip_q4_0_q8_0_gemm) at shapes of few output tiles: each work-group packs
 // its 64 weight rows and 64 tokens into records in LDS, one 8-block chunk at a
-// time (a lane per row, the row's chunk span realigned as the span pack does,
+// time (a lane per row, the row's chunk span realigned as the packs do,
 // in two halves on two waves per operand), and the four
 // waves fold their 32 x 32 tiles from there as gemm_tiles32 does from HBM.
 // Rows 16-byte aligned and a whole number of chunks (n a multiple of 256).
@@ -1587,86 +1617,70 @@ size_t tile_bytes(size_t nrows, size_t nb) {
   return (nrows + tcrv::kTG - 1) / tcrv::kTG * nb * tcrv::kTRec;
 }
 
+// Two ranges a work-group where one would make more than three a CU: more bytes in flight a
+// barrier (us, one range against two: 4096 x 4096 Q8_0 6.9 / 6.6, Q4_0 6.5 / 5.8; 11008 x
+// 4096 17.8 / 16.3, 14.7 / 13.0; but 1000 x 4096 3.4 / 3.6, 333 x 4096 2.7 / 3.2).  Not for the
+// two operands of a GEMM, whose records stay in the caches (4096^3 Q8_0: 163 / 167).
+constexpr size_t kPackManyMin = 768;
+size_t pack_ranges(size_t nrows, size_t nb) {
+  return (nrows + tcrv::kTG - 1) / tcrv::kTG * ((nb + tcrv::kPackSpan - 1) / tcrv::kPackSpan);
+}
+
+// One operand (q4: Q4_0 weights), streaming stores.
 int pack_tiles(size_t nrows, size_t nb, const uint8_t *src, size_t bx, uint8_t *dst,
-               hipStream_t st) {
+               hipStream_t st, bool q4 = false) {
   using namespace tcrv_host;
-  const size_t ngroups = (nrows + tcrv::kTG - 1) / tcrv::kTG;
-  size_t b0 = 0;  // blocks below b0 are packed by the span kernel
-  if (aligned16(src) && (nrows == 1 || bx % 16 == 0) && nb >= tcrv::kPackSpan) {
-    const size_t nspans = ngroups * (nb / tcrv::kPackSpan);
-    const size_t grid = (nspans * 64 + 255) / 256;
+  if (nb >= tcrv::kPackSpan) {
+    const size_t ranges = pack_ranges(nrows, nb);
+    const bool many = ranges >= kPackManyMin;
+    // a Q4_0 wave a range wants whole ranges and 16-byte aligned rows
+    const bool spans = q4 && many && nb % tcrv::kPackSpan == 0 && aligned16(src) && bx % 16 == 0;
+    const size_t grid = spans ? (ranges + 3) / 4 : many ? (ranges + 1) / 2 : ranges;
     if (grid > 0x7fffffffu)
       return TCRV_HIP_ERR_TOO_LARGE;
-    tcrv::pack_gemm_tiles_span<<<dim3(static_cast<unsigned>(grid)), dim3(256), 0, st>>>(
-        nrows, nb, src, bx, dst, nspans);
-    b0 = nb / tcrv::kPackSpan * tcrv::kPackSpan;
-  }
-  if (b0 < nb) {
-    const size_t nrec = ngroups * (nb - b0);
-    const size_t grid = (nrec * 64 + 255) / 256;
-    if (grid > 0x7fffffffu)
-      return TCRV_HIP_ERR_TOO_LARGE;
-    if (aligned4(src) && (nrows == 1 || bx % 4 == 0))
-      tcrv::pack_gemm_tiles<true><<<dim3(static_cast<unsigned>(grid)), dim3(256), 0, st>>>(
-          nrows, nb, src, bx, dst, b0, nrec);
+    auto run = [&](auto kernel) {
+      kernel<<<dim3(static_cast<unsigned>(grid)), dim3(256), 0, st>>>(nrows, nb, src, bx, dst,
+                                                                      ranges);
+    };
+    if (spans)
+      run(tcrv::pack_q4_tiles_span);
+    else if (many)
+      q4 ? run(tcrv::pack_tiles_ranges<true, 2>) : run(tcrv::pack_tiles_ranges<false, 2>);
     else
-      tcrv::pack_gemm_tiles<false><<<dim3(static_cast<unsigned>(grid)), dim3(256), 0, st>>>(
-          nrows, nb, src, bx, dst, b0, nrec);
+      q4 ? run(tcrv::pack_tiles_ranges<true, 1>) : run(tcrv::pack_tiles_ranges<false, 1>);
+    return launch_status();
   }
+  const size_t nrec = (nrows + tcrv::kTG - 1) / tcrv::kTG * nb, grid = (nrec + 3) / 4;
+  if (grid > 0x7fffffffu)
+    return TCRV_HIP_ERR_TOO_LARGE;
+  const dim3 g(static_cast<unsigned>(grid)), b(256);
+  if (q4)
+    tcrv::pack_q4_tiles<<<g, b, 0, st>>>(nrows, nb, src, bx, dst, nrec);
+  else
+    tcrv::pack_gemm_tiles<<<g, b, 0, st>>>(nrows, nb, src, bx, dst, nrec);
   return launch_status();
 }
 
-int pack_tiles_q4(size_t nrows, size_t nb, const uint8_t *src, size_t bx, uint8_t *dst,
-                  hipStream_t st) {
-  using namespace tcrv_host;
-  const size_t ngroups = (nrows + tcrv::kTG - 1) / tcrv::kTG;
-  size_t b0 = 0;  // blocks below b0 are packed by the span kernel
-  if (aligned16(src) && (nrows == 1 || bx % 16 == 0) && nb >= tcrv::kPackSpan) {
-    const size_t nspans = ngroups * (nb / tcrv::kPackSpan);
-    const size_t grid = (nspans * 64 + 255) / 256;
-    if (grid > 0x7fffffffu)
-      return TCRV_HIP_ERR_TOO_LARGE;
-    tcrv::pack_q4_tiles_span<<<dim3(static_cast<unsigned>(grid)), dim3(256), 0, st>>>(
-        nrows, nb, src, bx, dst, nspans);
-    b0 = nb / tcrv::kPackSpan * tcrv::kPackSpan;
-  }
-  if (b0 < nb) {
-    const size_t nrec = ngroups * (nb - b0);
-    const size_t grid = (nrec * 64 + 255) / 256;
-    if (grid > 0x7fffffffu)
-      return TCRV_HIP_ERR_TOO_LARGE;
-    tcrv::pack_q4_tiles<<<dim3(static_cast<unsigned>(grid)), dim3(256), 0, st>>>(
-        nrows, nb, src, bx, dst, b0, nrec);
-  }
-  return launch_status();
-}
-
-// Both operands of a GEMM (xq4: the weights vx are Q4_0): one launch of the span
-// kernel when every block of both is in an 8-block span of 16-byte aligned rows,
-// else one pack per operand.
+// Both operands of a GEMM (xq4: the weights vx are Q4_0): one launch from 8 blocks a row,
+// else one per operand.
 int pack_tiles_both(size_t nb, const uint8_t *vx, size_t bx, size_t nr, uint8_t *tx,
                     const uint8_t *vy, size_t by, size_t nc, uint8_t *ty, hipStream_t st,
                     bool xq4 = false) {
   using namespace tcrv_host;
-  auto spans_only = [&](const uint8_t *src, size_t stride, size_t nrows) {
-    return aligned16(src) && (nrows == 1 || stride % 16 == 0) && nb % tcrv::kPackSpan == 0;
-  };
-  if (nb == 0 || !spans_only(vx, bx, nr) || !spans_only(vy, by, nc)) {
-    const int rc = xq4 ? pack_tiles_q4(nr, nb, vx, bx, tx, st) : pack_tiles(nr, nb, vx, bx, tx, st);
+  if (nb < tcrv::kPackSpan) {
+    const int rc = pack_tiles(nr, nb, vx, bx, tx, st, xq4);
     return rc != TCRV_HIP_OK ? rc : pack_tiles(nc, nb, vy, by, ty, st);
   }
-  const size_t per_group = nb / tcrv::kPackSpan;
-  const tcrv::SpanOperand x{vx, bx, nr, (nr + tcrv::kTG - 1) / tcrv::kTG * per_group, tx};
-  const tcrv::SpanOperand y{vy, by, nc, (nc + tcrv::kTG - 1) / tcrv::kTG * per_group, ty};
-  const size_t grid = ((x.nspans + y.nspans) * 64 + 255) / 256;
+  const tcrv::SpanOperand x{vx, bx, nr, pack_ranges(nr, nb), tx};
+  const tcrv::SpanOperand y{vy, by, nc, pack_ranges(nc, nb), ty};
+  const size_t grid = x.nranges + y.nranges;
   if (grid > 0x7fffffffu)
     return TCRV_HIP_ERR_TOO_LARGE;
+  const dim3 g(static_cast<unsigned>(grid)), b(256);
   if (xq4)
-    tcrv::pack_gemm_tiles_span2<true>
-        <<<dim3(static_cast<unsigned>(grid)), dim3(256), 0, st>>>(nb, x, y);
+    tcrv::pack_tiles_ranges2<true><<<g, b, 0, st>>>(nb, x, y);
   else
-    tcrv::pack_gemm_tiles_span2<false>
-        <<<dim3(static_cast<unsigned>(grid)), dim3(256), 0, st>>>(nb, x, y);
+    tcrv::pack_tiles_ranges2<false><<<g, b, 0, st>>>(nb, x, y);
   return launch_status();
 }
 
@@ -1937,7 +1951,7 @@ int tcrv_hip_pack_q4_0_to_gemm_tiles(size_t nrows, size_t nb, const uint8_t *src
     return TCRV_HIP_ERR_MISALIGNED;
   if (nrows > 1 && bx < nb * tcrv::kQ4Bytes)
     return TCRV_HIP_ERR_BAD_SIZE;
-  return pack_tiles_q4(nrows, nb, src, bx, dst, as_stream(stream));
+  return pack_tiles(nrows, nb, src, bx, dst, as_stream(stream), true);
 }
 
 int tcrv_hip_q4_0_q8_0_gemm_tiles(size_t n, float *s, const uint8_t *tx, const uint8_t *ty,
