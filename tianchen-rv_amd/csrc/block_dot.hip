@@ -358,11 +358,131 @@ __global__ __launch_bounds__(kDdWaves * 64) void block_dot_half(float *s, size_t
     s[(p0 + fr) * os] = sumf;
 }
 
+// One token against rows of 130 to 512 blocks: the waves of a work-group (blockDim / 64,
+// 2 to 4) take `slice` consecutive blocks each of the same kRows rows and wave 0 folds.
+// What bounds the chunked kernels there: a wave loads, dots and folds 128 blocks
+// at a time, one load latency and one fold after another, with few waves at few rows, and a
+// last chunk of few blocks costs as much as a whole one.  Here all of K is in flight
+// at once, in slices of equal length, and only the ordered fold is serial.  Measured (us,
+// weights past the caches, before -> now): Q8_0 14336 x 512 6.65 -> 5.48, 5120 x 4096
+// 8.29 -> 7.27, 4160 x 14000 18.5 -> 14.2 (4.4 TB/s), 12544 x 14000 43.3 -> 39.1; Q4_0 14336 x
+// 512 6.49 -> 4.31, 9984 x 2048 6.76 -> 5.66.  From the caches 4160 x 14000 14.6 -> 11.8.
+template <DotFmt F, int kRows>
+__global__ __launch_bounds__(kDdWaves * 64) void gemv_long(unsigned nb, unsigned slice, float *s,
+                                                            size_t os, const uint8_t *vx,
+                                                            size_t bx, const uint8_t *vy,
+                                                            size_t nr) {
+  constexpr int kXBytes = F == DotFmt::kQ8Q8 ? kQ8Bytes : kQ4Bytes;
+  static_assert(kRows <= 4, "a DPP row folds each row");
+  __shared__ __align__(16) float2 tl[kRows][kDdWaves * kChunkBlocks + 8];
+  const unsigned w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const unsigned b = w * slice + 2 * l;
+  const size_t row0 = static_cast<size_t>(blockIdx.x) * kRows;
+  if (2 * l < slice && b < nb) {  // nb is even: the pair is whole or absent
+    uint32_t y0[8], y1[8], dy0, dy1;
+    load_q8_pair(vy + b * kQ8Bytes, y0, y1, dy0, dy1);
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      // rows past nr: computed, never stored
+      const uint8_t *x = vx + min(row0 + r, nr - 1) * bx + b * kXBytes;
+      int s0, s1;
+      uint32_t dx0, dx1;
+      if constexpr (F == DotFmt::kQ8Q8) {
+        uint32_t x0[8], x1[8];
+        load_q8_pair(x, x0, x1, dx0, dx1);
+        s0 = q8_q8_sumi(x0, y0);
+        s1 = q8_q8_sumi(x1, y1);
+      } else {
+        uint32_t x0[4], x1[4];
+        load_q4_pair(x, x0, x1, dx0, dx1);
+        s0 = q4_q8_sumi(x0, y0);
+        s1 = q4_q8_sumi(x1, y1);
+      }
+      const float2 t0 = fold_terms<F>(s0, dx0, dy0);
+      const float2 t1 = fold_terms<F>(s1, dx1, dy1);
+      *reinterpret_cast<float4 *>(&tl[r][b]) = make_float4(t0.x, t0.y, t1.x, t1.y);
+    }
+  }
+  // the last chunk's absent blocks: fma(0, 0, sumf) == sumf (sumf is never -0)
+  const unsigned nchunks = (nb + kChunkBlocks - 1) / kChunkBlocks;
+  const unsigned pad = nb + 2 * threadIdx.x;
+  if (pad < nchunks * kChunkBlocks) {
+#pragma unroll
+    for (int r = 0; r < kRows; ++r)
+      *reinterpret_cast<float4 *>(&tl[r][pad]) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+  __syncthreads();
+  if (w != 0)
+    return;
+  const unsigned fr = (l >> 4) % kRows, fp = l & (kDdLanes - 1);  // row folded, lane in chain
+  float sumf = 0.0f;
+  for (unsigned c = 0; c < nchunks; ++c) {
+    float ta[kDdTerms], tb[kDdTerms];
+#pragma unroll
+    for (int k = 0; k < kDdTerms; k += 2) {
+      const float4 v =
+          *reinterpret_cast<const float4 *>(&tl[fr][c * kChunkBlocks + fp * kDdTerms + k]);
+      ta[k] = v.x; tb[k] = v.y; ta[k + 1] = v.z; tb[k + 1] = v.w;
+    }
+    // the previous chunk's sum sits in the last lane of the fold row: seed lane 0
+    const float carry = __shfl(sumf, (l & ~(kDdLanes - 1)) + kDdLanes - 1);
+    sumf = fold_chain<kDdLanes, kDdTerms>(ta, tb, fp == 0 ? carry : 0.0f);
+  }
+  if (fp == kDdLanes - 1 && (l >> 4) < kRows && row0 + fr < nr)
+    s[(row0 + fr) * os] = sumf;
+}
+
 }  // namespace tcrv
 
 namespace tcrv_host {
 
 using tcrv::DotFmt;
+
+// Rows a work-group of gemv_long, or 0 where the chunked kernels are faster (Q8_0
+// block_dot_direct, Q4_0 gemv_q4_0_q8_0_direct) from memory or from the caches.
+// Measured both ways, gemv_long / chunked, us, "n x rows: memory; caches":
+//   - few rows leave the chunked kernels too few waves.  Q4_0: 5120 x 512 3.33/4.00; 3.03/3.76,
+//     14336 x 2048 7.98/8.25; 6.04/6.63, but 9984 x 4096 8.23/8.67; 6.65/5.83.  Q8_0: 14336 x 512
+//     5.48/6.65; 4.10/4.78, 9984 x 1024 5.76/5.93; 4.16/4.26, but 11008 x 1024 6.26/6.05; 4.17/4.24;
+//   - Q8_0, a second chunk of at most 64 blocks: 4160 x 2048 4.57/4.93; 3.88/4.14, 5120 x 14000
+//     16.6/19.2; 13.3/15.3, 6144 x 4096 8.17/8.77; 5.66/6.56 (2048 rows 5.58/5.52; 4.09/4.25);
+//     somewhat longer ones with one row a work-group: 6912 x 8000 12.9/14.5; 11.1/11.2, but 8192 x
+//     8000 14.6/15.7; 12.3/12.1, 9984 x 4096 11.6/12.2; 9.45/9.32;
+//   - Q8_0, a fourth chunk of at most 16: 12544 x 4096 14.7/15.2; 10.9/12.0, 12800 x 8000
+//     26.0/27.4; 18.3/19.4, but 13056 x 4096 15.9/15.6; 11.4/12.1.
+int gemv_long_rows(bool q4, size_t nb, size_t nr) {
+  if (nb <= static_cast<size_t>(tcrv::kChunkBlocks) ||
+      nb > static_cast<size_t>(tcrv::kDdWaves * tcrv::kChunkBlocks))
+    return 0;
+  if (q4)
+    return nr <= 2048 ? 2 : 0;
+  if (nr <= 768 || nb <= 160 || (nr <= 1024 && nb <= 320))
+    return 2;
+  if (nr < 4096)
+    return 0;
+  if (nb <= 192)
+    return 2;
+  return nb <= 216 || (nb > 384 && nb <= 400) ? 1 : 0;
+}
+
+template <DotFmt F>
+int launch_long(size_t nb, float *s, size_t os, const uint8_t *vx, size_t bx, const uint8_t *vy,
+                size_t nr, int rows, hipStream_t st) {
+  const unsigned waves = static_cast<unsigned>((nb + tcrv::kChunkBlocks - 1) / tcrv::kChunkBlocks);
+  const unsigned slice = static_cast<unsigned>((nb / 2 + waves - 1) / waves * 2);
+  const size_t groups = (nr + rows - 1) / rows;
+  if (groups > 0x7fffffffu)
+    return TCRV_HIP_ERR_TOO_LARGE;
+  auto run = [&](auto kernel) {
+    kernel<<<dim3(static_cast<unsigned>(groups)), dim3(waves * 64), 0, st>>>(
+        static_cast<unsigned>(nb), slice, s, os, vx, bx, vy, nr);
+  };
+  if (rows == 2)
+    run(tcrv::gemv_long<F, 2>);
+  else
+    run(tcrv::gemv_long<F, 1>);
+  return launch_status();
+}
 
 // The register-direct row pairs, one pair per wave when a stride is 0 (one row
 // shared by every pair), else two; rows of exactly 64 blocks two pairs per
@@ -391,6 +511,11 @@ int launch_direct_pairs(size_t nb, float *s, size_t os, const uint8_t *vx, size_
     tcrv::block_dot_half<F, 4><<<dim3(static_cast<unsigned>((npairs + per_q - 1) / per_q)), b, 0,
                                  st>>>(s, os, vx, bx, vy, by, npairs);
     return launch_status();
+  }
+  if (by == 0) {
+    const int rows = gemv_long_rows(F == DotFmt::kQ4Q8, nb, npairs);
+    if (rows > 0)
+      return launch_long<F>(nb, s, os, vx, bx, vy, npairs, rows, st);
   }
   if (shared)
     tcrv::block_dot_direct<F, 1><<<g, b, 0, st>>>(nb, s, os, vx, bx, vy, by, npairs);

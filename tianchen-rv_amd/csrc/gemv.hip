@@ -591,6 +591,7 @@ constexpr int kDirectRows = 4;
 // 1024 x 14336 7.53/8.28; past it, 3072 x 4096 3.80/3.37, 4096^2 3.94/3.70).
 constexpr size_t kDirectSmallRows = 2048;
 inline int direct_rows(size_t nr) { return nr <= kDirectSmallRows ? 2 : kDirectRows; }
+constexpr int kRowsByShape = 0;  // rows_per_wave of the shape-free entries
 
 // Rows of 64 blocks (n = 2048) run the half-wave kernel: with 8 rows per wave
 // from this many rows, where its work-groups fill the chip (us, against the
@@ -647,6 +648,11 @@ int gemv_q4_0_q8_0(size_t n, float *s, size_t os, const uint8_t *vx, size_t bx,
     return TCRV_HIP_ERR_BAD_SIZE;
   hipStream_t st = as_stream(stream);
   if (nb % 2 == 0 && aligned4(vx) && aligned4(vy) && (nr == 1 || bx % 4 == 0)) {
+    if (rows_per_wave == kRowsByShape) {
+      if (gemv_long_rows(true, nb, nr) > 0)
+        return q4_0_rows_direct(nb, s, os, vx, nr > 1 ? bx : 0, vy, 0, nr, stream);
+      rows_per_wave = direct_rows(nr);
+    }
     switch (rows_per_wave) {
     case 2: return launch_direct<2>(nb, s, os, vx, bx, vy, nr, st);
     case 8: return launch_direct<8>(nb, s, os, vx, bx, vy, nr, st);
@@ -782,7 +788,7 @@ int tcrv_hip_gemv_q4_0_q8_0(size_t n, float *s, const uint8_t *vx, size_t bx,
     return TCRV_HIP_OK;
   if (n / tcrv::kQK == 0)
     return tcrv_host::zero_outputs(s, nr, 1, 1, stream);
-  return tcrv_host::gemv_q4_0_q8_0(n, s, 1, vx, bx, vy, nr, stream, tcrv_host::direct_rows(nr));
+  return tcrv_host::gemv_q4_0_q8_0(n, s, 1, vx, bx, vy, nr, stream, tcrv_host::kRowsByShape);
 }
 
 int tcrv_hip_gemv_q4_0_q8_0_shaped(size_t n, float *s, const uint8_t *vx, size_t bx,
@@ -807,7 +813,7 @@ int tcrv_hip_q4_0_q8_0_gemm(size_t n, float *s, const uint8_t *vx, const uint8_t
   if (n / tcrv::kQK == 0)
     return tcrv_host::zero_outputs(s, nr * nc, bs, nc, stream);
   if (nc == 1)
-    return tcrv_host::gemv_q4_0_q8_0(n, s, bs, vx, bx, vy, nr, stream, tcrv_host::direct_rows(nr));
+    return tcrv_host::gemv_q4_0_q8_0(n, s, bs, vx, bx, vy, nr, stream, tcrv_host::kRowsByShape);
   if (!s || !vx || !vy)
     return TCRV_HIP_ERR_NULL_POINTER;
   if (!tcrv_host::aligned2(vx) || !tcrv_host::aligned2(vy) || (nr > 1 && (bx & 1u)) || (by & 1u))

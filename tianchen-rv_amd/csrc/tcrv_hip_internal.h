@@ -176,6 +176,9 @@ int zero_outputs(float *s, size_t count, size_t stride, size_t ncols, void *stre
 int q4_0_gemm_mfma(size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
                    size_t by, size_t nr, size_t nc, size_t bs, void *stream);
 
+// Rows a work-group of the K-split GEMV for long rows (block_dot.hip), 0 where it is not used.
+int gemv_long_rows(bool q4, size_t nb, size_t nr);
+
 // npairs register-direct block dots (block_dot.hip): s[p * os] = dot(vx + p*bx,
 // vy + p*by); a stride of 0 pairs every row of the other operand with one row
 // (the GEMM's nc = 1 and nr = 1 shapes).  TCRV_HIP_ERR_UNSUPPORTED for an odd
