@@ -1859,11 +1859,12 @@ bool ws_few_tokens(size_t nb, const uint8_t *vx, size_t bx, const uint8_t *vy, s
                    size_t nc) {
   return nc <= 24 && nb % 2 == 0 && aligned4(vx) && aligned4(vy) && bx % 4 == 0 && by % 4 == 0;
 }
-// And where the plain entry's few-tile kernel, which packs in LDS, beats a
-// separate pack: up to 448 of its work-groups at K up to 4096, past the 16 x 16
-// tiles' shapes (us, plain against the workspace path: 4096 x 128 x 4096 28.0 /
-// 30.6 Q8_0, 31.5 / 32.2 Q4_0; 14336 x 128 40.7 / 48.7, 42.0 / 45.9; but 4096 x
-// 512 41.8 / 39.9, 4096 x 128 x 14336 84.1 / 72.5).
+// And where the plain entry beats a separate pack: up to 448 work-groups of
+// gemm_rows_few at K up to 4096, past the 16 x 16 tiles' shapes (us, gemm_rows_few
+// against the workspace path: 14336 x 128 40.7 / 48.7 Q8_0, 42.0 / 45.9 Q4_0; but
+// 4096 x 512 41.8 / 39.9, 4096 x 128 x 14336 84.1 / 72.5).  The plain entry runs the
+// smaller of these shapes on gemm_rows16 (4096 x 128 x 4096 16.6 Q8_0, 18.4 Q4_0,
+// against 30.6 and 32.2 packed).
 bool ws_rows_few_first(size_t nb, const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by,
                        size_t nr, size_t nc) {
   return nb % tcrv::kFKB == 0 && nb <= 128 && aligned16(vx) && aligned16(vy) && bx % 16 == 0 &&

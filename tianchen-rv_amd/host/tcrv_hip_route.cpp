@@ -233,10 +233,9 @@ const tcrv_hip_schedule kSchedules[] = {
      "512 waves for 4096 rows leave half the SIMDs idle during the read"},
     // the tiled GEMMs: tokens per work-group tile; the entries pick per shape:
     // 64 x 64 tiles of one 32 x 32 tile a wave where 256 x 128 tiles would not
-    // fill one round of the CUs (at most 1024 work-groups), else 256 weight
-    // rows and the larger tile when its rounds of 256 work-groups x 15 are at
-    // most the smaller tile's rounds x 8 (one round of 256 x 256 tiles takes
-    // ~1.87 rounds of 256 x 128 ones)
+    // fill one round of the CUs (at most 1536 work-groups), else the tile of
+    // 256 x 256, 192 x 256 or 256 x 128 with the least rounds of 256
+    // work-groups x 32, 26 and 18 (a round's relative time)
     {"tcrv_rvv.q8_0_q8_0_gemm", TCRV_HIP_M_PREFILL, "gemm_tiles32", "work_group_tokens", 64, 0,
      nullptr, -1.0,
      "one 32x32 tile a wave, operands straight from the records; where few output tiles "
