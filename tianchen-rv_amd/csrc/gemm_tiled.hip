@@ -217,12 +217,12 @@ __device__ __forceinline__ void pack_range_rows(size_t nrows, size_t nb, const u
   }
 }
 
-template <bool kQ4, int kR>
+template <bool kQ4, int kR, bool kStream>
 __global__ __launch_bounds__(256) void pack_tiles_ranges(size_t nrows, size_t nb,
                                                          const uint8_t *src, size_t bx,
                                                          uint8_t *dst, size_t nranges) {
   __shared__ __align__(16) uint8_t raw[kR * kTG * kPackSpan * (kQ4 ? kQ4Bytes : kQ8Bytes)];
-  pack_range_rows<kQ4, true, kR>(nrows, nb, src, bx, dst, blockIdx.x, nranges, raw);
+  pack_range_rows<kQ4, kStream, kR>(nrows, nb, src, bx, dst, blockIdx.x, nranges, raw);
 }
 
 // Span `wave` of one Q4_0 operand with 16-byte aligned rows (bx % 16 == 0):
@@ -1626,7 +1626,7 @@ size_t pack_ranges(size_t nrows, size_t nb) {
   return (nrows + tcrv::kTG - 1) / tcrv::kTG * ((nb + tcrv::kPackSpan - 1) / tcrv::kPackSpan);
 }
 
-// One operand (q4: Q4_0 weights), streaming stores.
+// One operand (q4: Q4_0 weights).
 int pack_tiles(size_t nrows, size_t nb, const uint8_t *src, size_t bx, uint8_t *dst,
                hipStream_t st, bool q4 = false) {
   using namespace tcrv_host;
@@ -1634,7 +1634,14 @@ int pack_tiles(size_t nrows, size_t nb, const uint8_t *src, size_t bx, uint8_t *
     const size_t ranges = pack_ranges(nrows, nb);
     const bool many = ranges >= kPackManyMin;
     // a Q4_0 wave a range wants whole ranges and 16-byte aligned rows
-    const bool spans = q4 && many && nb % tcrv::kPackSpan == 0 && aligned16(src) && bx % 16 == 0;
+    const bool whole = nb % tcrv::kPackSpan == 0 && aligned16(src) && bx % 16 == 0;
+    const bool spans = q4 && many && whole;
+    // A GEMM that follows reads the records: streamed past the caches they cost it more
+    // than the pack gains where ranges overlap or rows lie off the lines (pack and GEMM,
+    // us, streamed / kept: 1030 x 2537 x 8864 97 / 86, 638 x 371 x 6720 Q4_0 29.3 / 27.6,
+    // 557 x 241 x 3648 Q4_0 18.2 / 16.7; the pack alone 7.2 / 8.7, 2.56 / 2.61, 2.37 / 2.35).  Whole ranges
+    // of aligned rows gain from streaming (above).
+    const bool stream = whole;
     const size_t grid = spans ? (ranges + 3) / 4 : many ? (ranges + 1) / 2 : ranges;
     if (grid > 0x7fffffffu)
       return TCRV_HIP_ERR_TOO_LARGE;
@@ -1644,10 +1651,18 @@ int pack_tiles(size_t nrows, size_t nb, const uint8_t *src, size_t bx, uint8_t *
     };
     if (spans)
       run(tcrv::pack_q4_tiles_span);
+    else if (stream && many)
+      q4 ? run(tcrv::pack_tiles_ranges<true, 2, true>)
+         : run(tcrv::pack_tiles_ranges<false, 2, true>);
+    else if (stream)
+      q4 ? run(tcrv::pack_tiles_ranges<true, 1, true>)
+         : run(tcrv::pack_tiles_ranges<false, 1, true>);
     else if (many)
-      q4 ? run(tcrv::pack_tiles_ranges<true, 2>) : run(tcrv::pack_tiles_ranges<false, 2>);
+      q4 ? run(tcrv::pack_tiles_ranges<true, 2, false>)
+         : run(tcrv::pack_tiles_ranges<false, 2, false>);
     else
-      q4 ? run(tcrv::pack_tiles_ranges<true, 1>) : run(tcrv::pack_tiles_ranges<false, 1>);
+      q4 ? run(tcrv::pack_tiles_ranges<true, 1, false>)
+         : run(tcrv::pack_tiles_ranges<false, 1, false>);
     return launch_status();
   }
   const size_t nrec = (nrows + tcrv::kTG - 1) / tcrv::kTG * nb, grid = (nrec + 3) / 4;
