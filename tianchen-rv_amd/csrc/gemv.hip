@@ -5,8 +5,8 @@
 // row ir and activation column col (RVVToEmitCBlockQuantLinear.cpp:1691-2121;
 // RVVOps.td:4147-4151).  The decode GEMV kernel below keeps that per-element
 // definition and its fold order, fma(fl((float)sumi*d_x), d_y, sumf) in
-// ascending block order; rows that are not 4-byte aligned and odd block counts
-// run gemm_batch.hip.
+// ascending block order; with more tokens, rows that are not 4-byte aligned and odd
+// block counts run gemm_batch.hip.
 #include "tcrv_hip_internal.h"
 
 namespace tcrv {
@@ -87,6 +87,117 @@ __device__ __forceinline__ int nibble_dot(const uint32_t q[4], const uint32_t y[
   }
   return acc;
 }
+
+// The decode GEMV over rows of an odd block count or off the 4-byte grid: a work-group of 4
+// waves owns 4 R rows; each wave stages its rows' chunk in LDS with 128-bit loads, all issued
+// before the first use, the activation chunk is staged once a work-group, and lane r < R folds
+// row r.  gemm_batch with one token moves a 16-column tile for one column (us, this kernel
+// against it: 4182 x 2336 6.04 / 7.51, 14000 x 2912 13.5 / 15.3, 5000 x 9120 17.2 / 19.2, 1509 x 1056
+// 3.90 / 4.01; but 14000 x 9120 38.0 / 36.0).
+constexpr int kGvWaves = 4;
+
+template <int kParity>
+__device__ __forceinline__ void gv_read_q8(const uint8_t *chunk, int b, uint32_t q[8],
+                                           uint32_t &d_bits) {
+  const uint32_t *w = reinterpret_cast<const uint32_t *>(chunk) + ((b * kQ8Bytes) >> 2);
+  uint32_t r[9];
+#pragma unroll
+  for (int k = 0; k < 9; ++k)
+    r[k] = w[k];
+  if constexpr (kParity == 0) {
+    d_bits = r[0] & 0xffffu;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      q[k] = funnel16(r[k], r[k + 1]);
+  } else {
+    d_bits = r[0] >> 16;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      q[k] = r[k + 1];
+  }
+}
+
+template <int kParity>
+__device__ __forceinline__ float gv_q4_term(const uint8_t *chunk, int b, const uint32_t qy[8]) {
+  const uint32_t *w = reinterpret_cast<const uint32_t *>(chunk) + ((b * kQ4Bytes) >> 2);
+  uint32_t r[5];
+#pragma unroll
+  for (int k = 0; k < 5; ++k)
+    r[k] = w[k];
+  uint32_t q[4], d_bits;
+  if constexpr (kParity == 0) {
+    d_bits = r[0] & 0xffffu;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      q[k] = funnel16(r[k], r[k + 1]);
+  } else {
+    d_bits = r[0] >> 16;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      q[k] = r[k + 1];
+  }
+  int acc = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    acc = sdot4(nibbles_to_i8x4(q[k]), qy[k], acc);
+    acc = sdot4(nibbles_to_i8x4(q[k] >> 4), qy[k + 4], acc);
+  }
+  return static_cast<float>(acc) * fp16_bits_to_f32(d_bits);
+}
+
+template <int R>
+__global__ __launch_bounds__(kGvWaves * 64) void gemv_q4_0_q8_0_kernel(
+    size_t nb, float *s, size_t os, const uint8_t *vx, size_t bx, const uint8_t *vy,
+    size_t nr) {
+  constexpr int kXRow = kGvChunk * kQ4Bytes + 16;  // 2320: 16-B multiple, +16 over-read pad
+  __shared__ __align__(16) uint8_t yl[kGvChunk * kQ8Bytes + 16];
+  __shared__ __align__(16) uint8_t xl[kGvWaves][R][kXRow];
+  __shared__ float tl[kGvWaves][R][kGvChunk + 1];
+  __shared__ float dyl[kGvChunk];
+
+  const int tid = threadIdx.x;
+  const int w = tid >> 6;
+  const int l = tid & 63;
+  const size_t row0 = (static_cast<size_t>(blockIdx.x) * kGvWaves + w) * R;
+  float sumf = 0.0f;  // lane r < R: running fold of row row0 + r
+
+  for (size_t c0 = 0; c0 < nb; c0 += kGvChunk) {
+    const int nbc = static_cast<int>(min(static_cast<size_t>(kGvChunk), nb - c0));
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const size_t row = min(row0 + r, nr - 1);  // rows past nr recompute row nr-1, unstored
+      copy_span_to_lds(xl[w][r], vx + row * bx + c0 * kQ4Bytes, nbc * kQ4Bytes, l, 64);
+    }
+    copy_span_to_lds(yl, vy + c0 * kQ8Bytes, nbc * kQ8Bytes, tid, kGvWaves * 64);
+    __syncthreads();
+    for (int b = tid; b < nbc; b += kGvWaves * 64)
+      dyl[b] = fp16_bits_to_f32(reinterpret_cast<const uint16_t *>(yl)[b * (kQ8Bytes / 2)]);
+    const int b0 = 2 * l, b1 = 2 * l + 1;
+    uint32_t qy0[8], qy1[8], dbits;
+    if (b0 < nbc)
+      gv_read_q8<0>(yl, b0, qy0, dbits);
+    if (b1 < nbc)
+      gv_read_q8<1>(yl, b1, qy1, dbits);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (b0 < nbc)
+        tl[w][r][b0] = gv_q4_term<0>(xl[w][r], b0, qy0);
+      if (b1 < nbc)
+        tl[w][r][b1] = gv_q4_term<1>(xl[w][r], b1, qy1);
+    }
+    __syncthreads();
+    if (l < R) {
+      const float *t = tl[w][l];
+#pragma unroll 8
+      for (int b = 0; b < nbc; ++b)
+        sumf = fmaf(t[b], dyl[b], sumf);
+    }
+    __syncthreads();
+  }
+  if (l < R && row0 + l < nr)
+    s[(row0 + l) * os] = sumf;
+}
+
 
 // kOneChunk: nb == kGvChunk exactly (n = 4096), so every lane owns a whole
 // block pair, there is one chunk and no carry between chunks.
@@ -591,6 +702,8 @@ constexpr int kDirectRows = 4;
 // 1024 x 14336 7.53/8.28; past it, 3072 x 4096 3.80/3.37, 4096^2 3.94/3.70).
 constexpr size_t kDirectSmallRows = 2048;
 inline int direct_rows(size_t nr) { return nr <= kDirectSmallRows ? 2 : kDirectRows; }
+// Rows per wave of the LDS-staged decode GEMV (odd nb or 2-byte aligned rows).
+constexpr int kGemvRows = 2;
 constexpr int kRowsByShape = 0;  // rows_per_wave of the shape-free entries
 
 // Rows of 64 blocks (n = 2048) run the half-wave kernel: with 8 rows per wave
@@ -659,7 +772,14 @@ int gemv_q4_0_q8_0(size_t n, float *s, size_t os, const uint8_t *vx, size_t bx,
     default: return launch_direct<kDirectRows>(nb, s, os, vx, bx, vy, nr, st);
     }
   }
-  return gemm_batch(true, nb, s, vx, bx, vy, 0, nr, 1, os, stream);
+  const size_t rows_per_wg = static_cast<size_t>(tcrv::kGvWaves) * kGemvRows;
+  const size_t grid = (nr + rows_per_wg - 1) / rows_per_wg;
+  if (grid > 0x7fffffffu)
+    return TCRV_HIP_ERR_TOO_LARGE;
+  tcrv::gemv_q4_0_q8_0_kernel<kGemvRows>
+      <<<dim3(static_cast<unsigned>(grid)), dim3(tcrv::kGvWaves * 64), 0, st>>>(
+          nb, s, os, vx, bx, vy, nr);
+  return launch_status();
 }
 
 template <bool kQ4, int kCols>
