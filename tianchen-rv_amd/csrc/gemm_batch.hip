@@ -32,6 +32,7 @@
 //   2110 -> 21.
 #include "tcrv_hip_internal.h"
 #include "mfma_fold.h"
+#include "tile_order.h"
 
 #include <type_traits>
 
@@ -105,14 +106,14 @@ __device__ __forceinline__ v4i bt_sums(uint32_t a0, uint32_t a1, uint32_t b0, ui
   return __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, v4i{}, 0, 0, 0);
 }
 
-// Work-group (x, group, z): row tile x + 8z, so the token groups of one row tile
-// run on one XCD (ids go round the 8 XCDs, x fastest), one after another.  At
+// Work-group (x, y, z): the tile of XCD x's slot (y, z), tile_order.h.  At
 // most four waves a SIMD: two work-groups of 8 waves a CU, one of 16.
 // kWide: row strides past 256 MB.
 template <bool kQ4, int kWaves, bool kWide>
 __global__ __launch_bounds__(kWaves * 64, 4) void gemm_batch(
-    const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by, size_t nr, size_t nb, unsigned nc,
-    float *s, size_t bs) {
+    uint32_t tiles, uint32_t tok_tiles, uint32_t inv, const uint8_t *vx,
+    size_t bx, const uint8_t *vy, size_t by, uint32_t nr, uint32_t nc, size_t nb, float *s,
+    size_t bs) {
   using Off = std::conditional_t<kWide, size_t, uint32_t>;  // of a row from the tile's first
   constexpr int kChunk = kWaves * kBtSlice;  // blocks
   constexpr int kXBlock = kQ4 ? kQ4Bytes : kQ8Bytes;
@@ -129,11 +130,11 @@ __global__ __launch_bounds__(kWaves * 64, 4) void gemm_batch(
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  const unsigned tile = blockIdx.x + 8 * blockIdx.z, group = blockIdx.y;
-  const size_t row0 = static_cast<size_t>(tile) * kBtRows;
-  if (row0 >= nr)
+  const TilePos tile = xcd_tile(tiles, tok_tiles, inv, blockIdx.x, blockIdx.y, blockIdx.z);
+  if (!tile.live)
     return;
-  const unsigned tok0 = group * kBtToks;
+  const size_t row0 = static_cast<size_t>(tile.tm) * kBtRows;
+  const unsigned tok0 = tile.tn * kBtToks;
   const int ntok = static_cast<int>(min(nc - tok0, static_cast<unsigned>(kBtToks)));
   uint8_t *region = lds + wave * kBtRegion;
 
@@ -316,21 +317,26 @@ namespace tcrv_host {
 
 int gemm_batch(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
                size_t by, size_t nr, size_t nc, size_t bs, void *stream) {
-  // a launch takes 65535 x 8 row tiles and 65535 token groups
-  constexpr size_t kMaxRows = static_cast<size_t>(65535) * 8 * tcrv::kBtRows;
-  constexpr size_t kMaxToks = static_cast<size_t>(65535) * tcrv::kBtToks;
+  // a launch takes 2^19 row tiles, then as many token groups as its tiles allow
+  constexpr size_t kMaxRows = (static_cast<size_t>(1) << 19) * tcrv::kBtRows;
   const bool wide = bx > 0x0fffffffu || by > 0x0fffffffu;
   hipStream_t st = as_stream(stream);
-  for (size_t r0 = 0; r0 < nr; r0 += kMaxRows)
-    for (size_t c0 = 0; c0 < nc; c0 += kMaxToks) {
-      const size_t rows = nr - r0 < kMaxRows ? nr - r0 : kMaxRows;
-      const size_t toks = nc - c0 < kMaxToks ? nc - c0 : kMaxToks;
-      const size_t tiles = (rows + tcrv::kBtRows - 1) / tcrv::kBtRows;
+  for (size_t r0 = 0; r0 < nr; r0 += kMaxRows) {
+    const size_t rows = nr - r0 < kMaxRows ? nr - r0 : kMaxRows;
+    const size_t tiles = (rows + tcrv::kBtRows - 1) / tcrv::kBtRows;
+    const size_t max_toks = (tcrv::kMaxTiles - 1) / tiles * tcrv::kBtToks;
+    for (size_t c0 = 0; c0 < nc; c0 += max_toks) {
+      const size_t toks = nc - c0 < max_toks ? nc - c0 : max_toks;
       const size_t groups = (toks + tcrv::kBtToks - 1) / tcrv::kBtToks;
-      const dim3 g(8, static_cast<unsigned>(groups), static_cast<unsigned>((tiles + 7) / 8));
+      tcrv::TileOrder o;
+      if (!tcrv::tile_order(tiles, groups, &o))
+        return TCRV_HIP_ERR_TOO_LARGE;
+      const dim3 g(tcrv::kXcds, o.slots_y, o.slots_z);
       auto run = [&](auto kernel, int waves) {
-        kernel<<<g, dim3(waves * 64), 0, st>>>(vx + r0 * bx, bx, vy + c0 * by, by, rows, nb,
-                                               static_cast<unsigned>(toks), s + r0 * bs + c0, bs);
+        kernel<<<g, dim3(waves * 64), 0, st>>>(o.total, o.tok_tiles, o.inv, vx + r0 * bx,
+                                               bx, vy + c0 * by, by, static_cast<uint32_t>(rows),
+                                               static_cast<uint32_t>(toks), nb,
+                                               s + r0 * bs + c0, bs);
       };
       // 16 waves where they hold all of K in one chunk and 8 would not, and a CU
       // has one work-group at most (4096 x 16 x 4096 Q4_0 6.2 against 6.8 us,
@@ -348,6 +354,7 @@ int gemm_batch(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const
       if (rc != TCRV_HIP_OK)
         return rc;
     }
+  }
   return TCRV_HIP_OK;
 }
 

@@ -22,6 +22,7 @@
 // waits; one chunk ahead instead of two cost 2 us.
 #include "tcrv_hip_internal.h"
 #include "mfma_fold.h"
+#include "tile_order.h"
 
 namespace tcrv {
 
@@ -39,12 +40,12 @@ struct RpStep {
   v16f dxy;
 };
 
-// Work-group (x, y, z): weight row tile x + 8z, token tile y, so the token tiles of one row
-// tile run on one XCD.  Weight groups past ngw and token groups past nga repeat the last one
+// Work-group (x, y, z): the tile of XCD x's slot (y, z), tile_order.h.  Weight groups past ngw and token groups past nga repeat the last one
 // (never stored).
 template <int kWM, int kWN>
 __global__ __launch_bounds__(kWM * kWN * 64, 2) void gemm_repack_mid(
-    size_t nb, float *s, const uint8_t *vx, const uint8_t *vy, size_t ngw, size_t nga, size_t bs,
+    uint32_t tiles, uint32_t tok_tiles, uint32_t inv, size_t nb,
+    const uint8_t *vx, const uint8_t *vy, size_t ngw, size_t nga, float *s, size_t bs,
     bool vec_out) {
   constexpr int kThreads = kWM * kWN * 64;
   constexpr int kBM = 32 * kWM, kBN = 32 * kWN, kRows = kBM + kBN;
@@ -63,10 +64,10 @@ __global__ __launch_bounds__(kWM * kWN * 64, 2) void gemm_repack_mid(
   const int wm = wave % kWM, wn = wave / kWM;
   const int li = lane & 31, h = lane >> 5;
   const size_t nrw = ngw * 16, ntok = nga * 4;
-  const size_t m0 = (blockIdx.x + 8 * static_cast<size_t>(blockIdx.z)) * kBM;
-  const size_t n0 = static_cast<size_t>(blockIdx.y) * kBN;
-  if (m0 >= nrw)
+  const TilePos tile = xcd_tile(tiles, tok_tiles, inv, blockIdx.x, blockIdx.y, blockIdx.z);
+  if (!tile.live)
     return;
+  const size_t m0 = static_cast<size_t>(tile.tm) * kBM, n0 = static_cast<size_t>(tile.tn) * kBN;
 
   // weight tasks: lane order (group, block, position quad, row quad)
   const uint8_t *wsrc[kWEach];
@@ -257,8 +258,6 @@ int gemm_repack_mid(size_t nb, float *s, const uint8_t *vx, const uint8_t *vy, s
   const size_t nrw = ngw * 16, ntok = nga * 4;
   const size_t nt = (ntok + 63) / 64;
   const size_t t64 = (nrw + 63) / 64 * nt, t128 = (nrw + 127) / 128 * nt;
-  if (nt > 65535 || (nrw + 63) / 64 > 65535u * 8)
-    return TCRV_HIP_ERR_UNSUPPORTED;
   // Rounds times a round's time at K 4096 (us): 256 work-groups of 128 x 64 outputs 33; of
   // 64 x 64, up to 256 26, then 512 (two a CU) 38; of the 256 x 128 kernel 87.
   // Measured, 64 / 128 / 256 rows: 4096 x 256 26.4 / 32.6 / 87, 4096 x 512 38.8 / 33.6 / 88,
@@ -268,14 +267,18 @@ int gemm_repack_mid(size_t nb, float *s, const uint8_t *vx, const uint8_t *vy, s
   const size_t c128 = (t128 + 255) / 256 * 33, c256 = (wide_tiles + 255) / 256 * 87;
   if (c256 < c64 && c256 < c128)
     return TCRV_HIP_ERR_UNSUPPORTED;
-  auto run = [&](auto kernel, size_t mt, int waves) {
-    kernel<<<dim3(8, static_cast<unsigned>(nt), static_cast<unsigned>((mt + 7) / 8)),
-             dim3(waves * 64), 0, as_stream(stream)>>>(nb, s, vx, vy, ngw, nga, bs, vec_out);
+  const bool rows64 = c64 <= c128;
+  tcrv::TileOrder o;
+  if (!tcrv::tile_order(rows64 ? (nrw + 63) / 64 : (nrw + 127) / 128, nt, &o))
+    return TCRV_HIP_ERR_UNSUPPORTED;
+  auto run = [&](auto kernel, int waves) {
+    kernel<<<dim3(tcrv::kXcds, o.slots_y, o.slots_z), dim3(waves * 64), 0, as_stream(stream)>>>(
+        o.total, o.tok_tiles, o.inv, nb, vx, vy, ngw, nga, s, bs, vec_out);
   };
-  if (c64 <= c128)
-    run(tcrv::gemm_repack_mid<2, 2>, (nrw + 63) / 64, 4);
+  if (rows64)
+    run(tcrv::gemm_repack_mid<2, 2>, 4);
   else
-    run(tcrv::gemm_repack_mid<4, 2>, (nrw + 127) / 128, 8);
+    run(tcrv::gemm_repack_mid<4, 2>, 8);
   return launch_status();
 }
 

@@ -25,6 +25,7 @@
 // thirds of the time (Q4_0) and a wave waits a third of it, for barriers mostly.
 #include "tcrv_hip_internal.h"
 #include "mfma_fold.h"
+#include "tile_order.h"
 
 namespace tcrv {
 
@@ -105,12 +106,12 @@ __device__ __forceinline__ v4f r16_scales(uint32_t a, uint32_t b) {
   return __builtin_amdgcn_mfma_f32_16x16x16f16(ha, hb, v4f{}, 0, 0, 0);
 }
 
-// Work-group (x, y, z): row tile x + 8z, token tile y, so the token tiles of one row tile run
-// on one XCD, one after another.
+// Work-group (x, y, z): the tile of XCD x's slot (y, z), tile_order.h.
 template <bool kQ4, int kWM>
 __global__ __launch_bounds__(kWM * 2 * 64, 2) void gemm_rows16(
-    const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by, size_t nr, size_t nb, size_t nc,
-    float *s, size_t bs) {
+    uint32_t tiles, uint32_t tok_tiles, uint32_t inv, const uint8_t *vx,
+    size_t bx, const uint8_t *vy, size_t by, uint32_t nr, uint32_t nc, size_t nb, float *s,
+    size_t bs) {
   constexpr int kWN = 2;
   constexpr int kCB = kR16Chunk;
   constexpr int kThreads = kWM * kWN * 64;
@@ -133,10 +134,10 @@ __global__ __launch_bounds__(kWM * 2 * 64, 2) void gemm_rows16(
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % kWM, wn = wave / kWM;
-  const size_t m0 = (blockIdx.x + 8 * static_cast<size_t>(blockIdx.z)) * kBM;
-  const size_t n0 = static_cast<size_t>(blockIdx.y) * kBN;
-  if (m0 >= nr)
+  const TilePos tile = xcd_tile(tiles, tok_tiles, inv, blockIdx.x, blockIdx.y, blockIdx.z);
+  if (!tile.live)
     return;
+  const size_t m0 = static_cast<size_t>(tile.tm) * kBM, n0 = static_cast<size_t>(tile.tn) * kBN;
   const uint32_t xlast = static_cast<uint32_t>(min(static_cast<size_t>(kBM), nr - m0)) - 1;
   const uint32_t ylast = static_cast<uint32_t>(min(static_cast<size_t>(kBN), nc - n0)) - 1;
   const uint8_t *xbase = vx + m0 * bx, *ybase = vy + n0 * by;
@@ -300,8 +301,8 @@ namespace tcrv_host {
 
 int gemm_rows16(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
                 size_t by, size_t nr, size_t nc, size_t bs, void *stream) {
-  // 32-bit row offsets within a work-group's 64 rows; the grid's y and z
-  if (bx > 0x03ffffffu || by > 0x03ffffffu || nc > 65535u * 32 || nr > 65535u * 8 * 32)
+  // 32-bit row offsets within a work-group's 64 rows, and row and token counts
+  if (bx > 0x03ffffffu || by > 0x03ffffffu || nr > 0xffffffffu || nc > 0xffffffffu)
     return TCRV_HIP_ERR_UNSUPPORTED;
   // 32-row work-groups while they fit one a CU, and for two to three rounds of them
   // (us, Q4_0 / Q8_0, 32 against 64 rows: 4096 x 64 13.3 / 12.4 against 18.2 / 16.3,
@@ -310,9 +311,14 @@ int gemm_rows16(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, cons
   const size_t w32 = (nr + 31) / 32 * ((nc + 31) / 32);
   const bool rows32 = w32 <= 256 || (w32 > 512 && w32 <= 768);
   const size_t mt = rows32 ? (nr + 31) / 32 : (nr + 63) / 64;
-  const dim3 g(8, static_cast<unsigned>((nc + 31) / 32), static_cast<unsigned>((mt + 7) / 8));
+  tcrv::TileOrder o;
+  if (!tcrv::tile_order(mt, (nc + 31) / 32, &o))
+    return TCRV_HIP_ERR_UNSUPPORTED;
+  const dim3 g(tcrv::kXcds, o.slots_y, o.slots_z);
   auto run = [&](auto kernel, int waves) {
-    kernel<<<g, dim3(waves * 64), 0, as_stream(stream)>>>(vx, bx, vy, by, nr, nb, nc, s, bs);
+    kernel<<<g, dim3(waves * 64), 0, as_stream(stream)>>>(
+        o.total, o.tok_tiles, o.inv, vx, bx, vy, by, static_cast<uint32_t>(nr),
+        static_cast<uint32_t>(nc), nb, s, bs);
   };
   if (rows32)
     q4 ? run(tcrv::gemm_rows16<true, 2>, 4) : run(tcrv::gemm_rows16<false, 2>, 4);
