@@ -3,6 +3,7 @@ the library's own host code runs in a child process against tests/launch_recorde
 place of the HIP runtime, so the rules that choose a kernel are the shipped ones and not a
 copy of them."""
 import ctypes
+import functools
 import json
 import os
 import subprocess
@@ -24,14 +25,19 @@ class Launch:
         return f"{self.name}{self.grid}x{self.block}"
 
 
+@functools.lru_cache(None)
+def _recorder():
+    tmp = tempfile.TemporaryDirectory()
+    lib = os.path.join(tmp.name, "recorder.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-fPIC", "-shared",
+                    os.path.join(HERE, "launch_recorder.cpp"), "-o", lib], check=True)
+    return tmp, lib  # the folder goes with the process
+
+
 def replay(calls):
     """calls: [(symbol, arguments without the stream)] -> [(status, [Launch])]."""
-    with tempfile.TemporaryDirectory() as tmp:
-        lib = os.path.join(tmp, "recorder.so")
-        subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-fPIC", "-shared",
-                        os.path.join(HERE, "launch_recorder.cpp"), "-o", lib], check=True)
-        out = subprocess.run([sys.executable, os.path.abspath(__file__), lib],
-                             input=json.dumps(calls), capture_output=True, text=True)
+    out = subprocess.run([sys.executable, os.path.abspath(__file__), _recorder()[1]],
+                         input=json.dumps(calls), capture_output=True, text=True)
     assert out.returncode == 0, out.stderr[-2000:]
     return [(status, [Launch(*x) for x in xs]) for status, xs in json.loads(out.stdout)]
 

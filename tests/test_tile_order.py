@@ -29,7 +29,7 @@ int main() {
       size_t live = 0;
       for (unsigned z = 0; z < o.slots_z; ++z)
         for (unsigned y = 0; y < o.slots_y; ++y) {
-          const TilePos p = xcd_tile(o.total, o.tok_tiles, o.inv, x, y, z);
+          const TilePos p = xcd_tile(o.total, t, o.inv, x, y, z);
           if (!p.live) continue;
           ++live;
           if (p.tm >= r || p.tn >= t || seen[static_cast<size_t>(p.tm) * t + p.tn]++) return 2;

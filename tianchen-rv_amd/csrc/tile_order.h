@@ -26,14 +26,14 @@ constexpr uint32_t kSlotsY = 512;
 // A launch takes fewer tiles than this (z is 65535 at most).
 constexpr size_t kMaxTiles = static_cast<size_t>(kXcds) * kSlotsY * 65535;
 
-// Kernel arguments of the order, each a dword of its own and first in the list: the command
-// processor preloads them, where a division or a read of gridDim would hold back a wave's first
-// loads (0.1-0.25 us of a 3-10 us kernel).
+// The order of a launch.  The kernels take total and inv as their first arguments and count the
+// token tiles from their own: what a wave needs before its first loads stays within the 14
+// argument dwords that the command processor preloads (an argument past them, or a read of
+// gridDim, is a scalar load that the loads wait for: 0.1-0.4 us of a 3-10 us kernel).
 struct TileOrder {
-  uint32_t total;      // tiles
-  uint32_t tok_tiles;  // token tiles of a row tile
-  uint32_t inv;        // 2^32 / tok_tiles, rounded down (2^32 - 1 for one)
-  uint32_t slots_y, slots_z;  // the grid's y and z, not passed on
+  uint32_t total;             // tiles
+  uint32_t inv;               // 2^32 / token tiles, rounded down (2^32 - 1 for one)
+  uint32_t slots_y, slots_z;  // the grid's y and z
 };
 
 struct TilePos {
@@ -46,7 +46,6 @@ inline bool tile_order(size_t row_tiles, size_t tok_tiles, TileOrder *o) {
   if (row_tiles >= kMaxTiles || tok_tiles >= kMaxTiles || row_tiles * tok_tiles >= kMaxTiles)
     return false;
   o->total = static_cast<uint32_t>(row_tiles * tok_tiles);
-  o->tok_tiles = static_cast<uint32_t>(tok_tiles);
   o->inv = tok_tiles == 1 ? 0xffffffffu : static_cast<uint32_t>((1ull << 32) / tok_tiles);
   const uint32_t slots = (o->total + kXcds - 1) / kXcds;  // the longest run
   o->slots_y = slots < kSlotsY ? slots : kSlotsY;
