@@ -1,0 +1,36 @@
+"""Which kernel an entry runs at a size: the shipped rules, replayed without a GPU
+(tests/launches.py)."""
+import pytest
+
+import launches
+
+# quant, entry, weight rows, tokens, n, keyword arguments of gemm_call, kernel
+SIZES = [
+    # half-empty 64-row tiles: as many 32-row work-groups
+    ("q8_0", "plain", 31, 9893, 3840, {}, "gemm_rows16<false, 2>"),
+    ("q4_0", "plain", 2317, 211, 4960, {}, "gemm_rows16<true, 2>"),
+    ("q8_0", "plain", 212, 4169, 2176, {}, "gemm_rows16<false, 2>"),
+    ("q4_0", "plain", 4096, 128, 4096, {}, "gemm_rows16<true, 4>"),
+    ("q8_0", "plain", 4096, 64, 4096, {}, "gemm_rows16<false, 2>"),
+    # few outputs, where gemm_rows_few serves
+    ("q4_0", "plain", 4096, 192, 4096, {}, "gemm_rows16<true, 2>"),
+    ("q8_0", "plain", 4096, 192, 4096, {}, "gemm_rows_few<false>"),
+    ("q8_0", "plain", 6457, 75, 512, {}, "gemm_rows16<false, 2>"),
+    ("q8_0", "plain", 4894, 127, 256, {}, "gemm_rows_few<false>"),
+    ("q4_0", "plain", 1166, 596, 256, {}, "gemm_rows_few<true>"),
+    # few weight rows and many tokens, K no multiple of 256
+    ("q8_0", "plain", 190, 8881, 10432, {}, "gemm_occ<false>"),
+    ("q4_0", "plain", 120, 14581, 960, {}, "gemm_occ<true>"),
+    ("q8_0", "plain", 154, 7280, 2880, {}, "gemm_rows16<false, 2>"),
+    # against the 256-row tiles
+    ("q8_0", "plain", 6192, 244, 640, {}, "gemm_wide<false>"),
+    ("q4_0", "plain", 977, 1672, 320, {}, "gemm_rows16<true, 4>"),
+    ("q4_0", "plain", 4096, 512, 4160, {}, "gemm_rows16<true, 4>"),
+    ("q4_0", "plain", 4096, 1000, 4160, {}, "gemm_wide<true>"),
+]
+
+
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: "-".join(map(str, s[:5])))
+def test_kernel_of_a_size(size):
+    *call, kw, want = size
+    assert launches.kernels([launches.gemm_call(*call, **kw)])[0][-1] == want

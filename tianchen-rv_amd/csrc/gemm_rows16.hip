@@ -300,17 +300,27 @@ __global__ __launch_bounds__(kWM * 2 * 64, 2) void gemm_rows16(
 
 namespace tcrv_host {
 
+// 32- or 64-row work-groups, by rounds of 256 (a CU holds one or two of either).  Measured over
+// 400 sizes, us a block of K beyond 1-3 us, Q4_0 / Q8_0: 32 rows, 1 to 4 rounds 0.085 / 0.082,
+// 0.135 / 0.116, 0.193 / 0.193, 0.257 / 0.245, 7 rounds 0.43 / 0.41; 64 rows 0.125 / 0.113,
+// 0.221 / 0.229, 0.337 / 0.373, 4 rounds 0.40 / 0.44.  Where a last 64-row tile is half empty the
+// two have nearly as many work-groups: 31 x 9893 x 3840 Q8_0 24.5 / 31.9, 212 x 4169 x 2176 Q8_0
+// 24.0 / 31.9, 2317 x 211 x 4960 Q4_0 26.0 / 37.6.
+bool rows16_by_32(bool q4, size_t w32, size_t w64) {
+  if (w64 <= 256)
+    return w32 <= 256;
+  if (w64 <= 512)
+    return w32 <= 768;
+  return w32 <= (q4 ? 1024 : 1792);
+}
+
 int gemm_rows16(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
                 size_t by, size_t nr, size_t nc, size_t bs, void *stream) {
   // 32-bit row offsets within a work-group's 64 rows, and row and token counts
   if (bx > 0x03ffffffu || by > 0x03ffffffu || nr > 0xffffffffu || nc > 0xffffffffu)
     return TCRV_HIP_ERR_UNSUPPORTED;
-  // 32-row work-groups while they fit one a CU, and for two to three rounds of them
-  // (us, Q4_0 / Q8_0, 32 against 64 rows: 4096 x 64 13.3 / 12.4 against 18.2 / 16.3,
-  // 4096 x 128 18.8 / 17.1 against 18.4 / 16.6, 4096 x 192 28.1 / 26.0 against 29.5 /
-  // 31.1, 4096 x 256 36 / 33 against 30 / 31.6)
-  const size_t w32 = (nr + 31) / 32 * ((nc + 31) / 32);
-  const bool rows32 = w32 <= 256 || (w32 > 512 && w32 <= 768);
+  const size_t w32 = (nr + 31) / 32 * ((nc + 31) / 32), w64 = (nr + 63) / 64 * ((nc + 31) / 32);
+  const bool rows32 = rows16_by_32(q4, w32, w64);
   const size_t mt = rows32 ? (nr + 31) / 32 : (nr + 63) / 64;
   tcrv::TileOrder o;
   if (!tcrv::tile_order(mt, (nc + 31) / 32, &o))
@@ -328,14 +338,34 @@ int gemm_rows16(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, cons
   return launch_status();
 }
 
+// Whether gemm_rows16 runs a shape of 4-byte aligned rows.  Measured over the same sizes, us:
+//   - against gemm_rows_few, where that serves: up to two rounds of 32-row work-groups (4096 x 128
+//     x 4096 18.4 / 16.6 against 31.0 / 26.7), and three of Q4_0 (0.193 against 0.214 a block) but
+//     for K 256, half a chunk (1166 x 596 5.8 / 5.0); three of Q8_0 cost as much (0.193 against 0.179)
+//     but for few whole chunks (6457 x 75 x 512 5.5 / 6.1, 2659 x 258 x 1536 11.5 / 12.2, but
+//     4894 x 127 x 256 5.2 / 4.7, 107 x 4937 x 1792 14.6 / 13.5);
+//   - else, under 256 weight rows, against the 128 x 128 tiles (one round 0.40 / 0.36 a block): three
+//     rounds of 64-row work-groups (Q4_0), five of 32-row ones (Q8_0) (190 x 8881 x 10432 Q8_0
+//     138 / 125, 120 x 14581 x 960 Q4_0 19.7 / 17.4);
+//   - else against the 256-row tiles (0.67 / 0.63 a block, few as they may be): four rounds of
+//     64-row work-groups (K 4160, 4096 x 512 61 / 70 against 101 / 93.6, 4096 x 1000 118 / 138
+//     against 101 / 92.5), two of Q8_0 at K under 1024 (6192 x 244 x 640 20.2 / 16.9; Q4_0 977 x
+//     1672 x 320 9.9 / 12.3).
+bool rows16_first(bool q4, size_t nb, size_t nr, size_t nc, bool few_serves) {
+  const size_t w32 = (nr + 31) / 32 * ((nc + 31) / 32), w64 = (nr + 63) / 64 * ((nc + 31) / 32);
+  if (few_serves)
+    return w32 <= 512 || (w32 <= 768 && (q4 ? nb >= 16 : nb % 16 == 0 && nb <= 48));
+  if (nr < 256)
+    return q4 ? w64 <= 768 : w32 <= 1280;
+  return nc <= 64 || w64 <= (!q4 && nb < 32 ? 512 : 1024);
+}
+
 int gemm_small(bool q4, bool rows4, size_t nb, float *s, const uint8_t *vx, size_t bx,
                const uint8_t *vy, size_t by, size_t nr, size_t nc, size_t bs, void *stream) {
   if (batch_first(rows4, nb, nr, nc))
     return gemm_batch(q4, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
-  const size_t w32 = (nr + 31) / 32 * ((nc + 31) / 32), w64 = (nr + 63) / 64 * ((nc + 31) / 32);
-  if (nr > 1 && nc > 4 &&
-      (!rows4 || w32 <= 768 ||
-       ((w64 <= 1024 || nc <= 64) && !rows_few_serves(nb, vx, bx, vy, by, nr, nc)))) {
+  if (nr > 1 && nc > 4 && (!rows4 || rows16_first(q4, nb, nr, nc,
+                                                  rows_few_serves(nb, vx, bx, vy, by, nr, nc)))) {
     const int st = gemm_rows16(q4, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
     if (st != TCRV_HIP_ERR_UNSUPPORTED)
       return st;

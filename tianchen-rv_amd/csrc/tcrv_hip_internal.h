@@ -211,18 +211,14 @@ inline bool batch_first(bool rows4, size_t nb, size_t nr, size_t nc) {
 
 // The GEMMs with one 16 x 16 tile a wave, a work-group's rows shared through LDS
 // (gemm_rows16.hip): any 2-byte aligned rows, any block count.
-// TCRV_HIP_ERR_UNSUPPORTED for row strides past 64 MB (and over 2 million tokens
-// or 16 million rows).
+// TCRV_HIP_ERR_UNSUPPORTED for row strides past 64 MB (and for 2^28 tiles or 2^32 rows).
 int gemm_rows16(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
                 size_t by, size_t nr, size_t nc, size_t bs, void *stream);
 
 // The plain-row GEMMs of few outputs and those of rows that are not 4-byte aligned:
 // gemm_batch or gemm_rows16, or TCRV_HIP_ERR_UNSUPPORTED where the kernels for
-// 4-byte aligned rows are faster (the multi-column GEMVs; gemm_rows_few past three
-// rounds of 32-row work-groups: 4096 x 192 x 4096 31.2 / 26.8 against 28.1 / 26.0
-// us, 4096 x 256 31.4 / 27.0 against 29.9 / 31.6; where it does not serve the rows,
-// the 256-row tiles past 1024 64-row work-groups: K 4160, 4096 x 512 101 / 93.6
-// against 61 / 70, 4096 x 1000 101 / 92.5 against 118 / 138).
+// 4-byte aligned rows are faster (the multi-column GEMVs; past the rule of rows16_first in
+// gemm_rows16.hip gemm_rows_few, or the 256- and 128-row tiles).
 int gemm_small(bool q4, bool rows4, size_t nb, float *s, const uint8_t *vx, size_t bx,
                const uint8_t *vy, size_t by, size_t nr, size_t nc, size_t bs, void *stream);
 
