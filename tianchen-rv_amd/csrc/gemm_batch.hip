@@ -111,7 +111,7 @@ __device__ __forceinline__ v4i bt_sums(uint32_t a0, uint32_t a1, uint32_t b0, ui
 // kWide: row strides past 256 MB.
 template <bool kQ4, int kWaves, bool kWide>
 __global__ __launch_bounds__(kWaves * 64, 4) void gemm_batch(
-    uint32_t tiles, uint32_t inv, const uint8_t *vx,
+    uint32_t units, uint32_t inv, const uint8_t *vx,
     size_t bx, const uint8_t *vy, size_t by, uint32_t nr, uint32_t nc, size_t nb, float *s,
     size_t bs) {
   using Off = std::conditional_t<kWide, size_t, uint32_t>;  // of a row from the tile's first
@@ -130,8 +130,9 @@ __global__ __launch_bounds__(kWaves * 64, 4) void gemm_batch(
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  const TilePos tile =
-      xcd_tile(tiles, (nc + kBtToks - 1) / kBtToks, inv, blockIdx.x, blockIdx.y, blockIdx.z);
+  const TilePos tile = xcd_tile(units, (nr + kBtRows - 1) / kBtRows,
+                                (nc + kBtToks - 1) / kBtToks, inv, blockIdx.x, blockIdx.y,
+                                blockIdx.z);
   if (!tile.live)
     return;
   const size_t row0 = static_cast<size_t>(tile.tm) * kBtRows;
@@ -334,7 +335,7 @@ int gemm_batch(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const
         return TCRV_HIP_ERR_TOO_LARGE;
       const dim3 g(tcrv::kXcds, o.slots_y, o.slots_z);
       auto run = [&](auto kernel, int waves) {
-        kernel<<<g, dim3(waves * 64), 0, st>>>(o.total, o.inv, vx + r0 * bx,
+        kernel<<<g, dim3(waves * 64), 0, st>>>(o.units, o.inv, vx + r0 * bx,
                                                bx, vy + c0 * by, by, static_cast<uint32_t>(rows),
                                                static_cast<uint32_t>(toks), nb,
                                                s + r0 * bs + c0, bs);

@@ -44,7 +44,7 @@ struct RpStep {
 // (never stored).
 template <int kWM, int kWN>
 __global__ __launch_bounds__(kWM * kWN * 64, 2) void gemm_repack_mid(
-    uint32_t tiles, uint32_t inv, size_t nb,
+    uint32_t units, uint32_t inv, size_t nb,
     const uint8_t *vx, const uint8_t *vy, size_t ngw, size_t nga, float *s, size_t bs,
     bool vec_out) {
   constexpr int kThreads = kWM * kWN * 64;
@@ -64,8 +64,9 @@ __global__ __launch_bounds__(kWM * kWN * 64, 2) void gemm_repack_mid(
   const int wm = wave % kWM, wn = wave / kWM;
   const int li = lane & 31, h = lane >> 5;
   const size_t nrw = ngw * 16, ntok = nga * 4;
-  const TilePos tile =
-      xcd_tile(tiles, static_cast<uint32_t>((ntok + kBN - 1) / kBN), inv, blockIdx.x, blockIdx.y, blockIdx.z);
+  const TilePos tile = xcd_tile(units, static_cast<uint32_t>((nrw + kBM - 1) / kBM),
+                                static_cast<uint32_t>((ntok + kBN - 1) / kBN), inv, blockIdx.x, blockIdx.y,
+                                blockIdx.z);
   if (!tile.live)
     return;
   const size_t m0 = static_cast<size_t>(tile.tm) * kBM, n0 = static_cast<size_t>(tile.tn) * kBN;
@@ -274,7 +275,7 @@ int gemm_repack_mid(size_t nb, float *s, const uint8_t *vx, const uint8_t *vy, s
     return TCRV_HIP_ERR_UNSUPPORTED;
   auto run = [&](auto kernel, int waves) {
     kernel<<<dim3(tcrv::kXcds, o.slots_y, o.slots_z), dim3(waves * 64), 0, as_stream(stream)>>>(
-        o.total, o.inv, nb, vx, vy, ngw, nga, s, bs, vec_out);
+        o.units, o.inv, nb, vx, vy, ngw, nga, s, bs, vec_out);
   };
   if (rows64)
     run(tcrv::gemm_repack_mid<2, 2>, 4);

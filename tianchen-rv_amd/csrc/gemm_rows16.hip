@@ -109,7 +109,7 @@ __device__ __forceinline__ v4f r16_scales(uint32_t a, uint32_t b) {
 // Work-group (x, y, z): the tile of XCD x's slot (y, z), tile_order.h.
 template <bool kQ4, int kWM>
 __global__ __launch_bounds__(kWM * 2 * 64, 2) void gemm_rows16(
-    uint32_t tiles, uint32_t inv, const uint8_t *vx,
+    uint32_t units, uint32_t inv, const uint8_t *vx,
     size_t bx, const uint8_t *vy, size_t by, uint32_t nr, uint32_t nc, size_t nb, float *s,
     size_t bs) {
   constexpr int kWN = 2;
@@ -134,8 +134,9 @@ __global__ __launch_bounds__(kWM * 2 * 64, 2) void gemm_rows16(
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % kWM, wn = wave / kWM;
-  const TilePos tile =
-      xcd_tile(tiles, (nc + kBN - 1) / kBN, inv, blockIdx.x, blockIdx.y, blockIdx.z);
+  const TilePos tile = xcd_tile(units, (nr + kBM - 1) / kBM,
+                                (nc + kBN - 1) / kBN, inv, blockIdx.x, blockIdx.y,
+                                blockIdx.z);
   if (!tile.live)
     return;
   const size_t m0 = static_cast<size_t>(tile.tm) * kBM, n0 = static_cast<size_t>(tile.tn) * kBN;
@@ -328,7 +329,7 @@ int gemm_rows16(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, cons
   const dim3 g(tcrv::kXcds, o.slots_y, o.slots_z);
   auto run = [&](auto kernel, int waves) {
     kernel<<<g, dim3(waves * 64), 0, as_stream(stream)>>>(
-        o.total, o.inv, vx, bx, vy, by, static_cast<uint32_t>(nr),
+        o.units, o.inv, vx, bx, vy, by, static_cast<uint32_t>(nr),
         static_cast<uint32_t>(nc), nb, s, bs);
   };
   if (rows32)
