@@ -114,12 +114,14 @@ __device__ __forceinline__ float2 block_terms(const uint8_t *xc, const uint8_t *
   }
 }
 
-// One wave (64 threads) per pair p: x row p, y row p, output s[p].
+// One wave (64 threads) per pair p: x row p, y row p, output s[p].  kGrid: x row blockIdx.y,
+// y row blockIdx.x, output s[blockIdx.y * bs + blockIdx.x] (the reference GEMM's loop nest).
 // kSums: write sumi[p*nb + b] instead of the fold.
-template <DotFmt F, bool kSums>
+template <DotFmt F, bool kSums, bool kGrid = false>
 __global__ __launch_bounds__(64) void block_dot_pairs(size_t nb, float *s, int32_t *sums,
                                                       const uint8_t *vx, size_t bx,
-                                                      const uint8_t *vy, size_t by) {
+                                                      const uint8_t *vy, size_t by,
+                                                      size_t bs) {
   constexpr int kXBytes = F == DotFmt::kQ8Q8 ? kQ8Bytes : kQ4Bytes;
   // +16: the last even block's 9th dword (or 5th) reads 2 bytes past its end.
   __shared__ __align__(16) uint8_t xl[kChunkBlocks * kXBytes + 16];
@@ -127,7 +129,8 @@ __global__ __launch_bounds__(64) void block_dot_pairs(size_t nb, float *s, int32
   __shared__ float2 terms[kChunkBlocks];
 
   const size_t p = blockIdx.x;
-  const uint8_t *xrow = vx + p * bx;
+  const size_t xr = kGrid ? blockIdx.y : p;
+  const uint8_t *xrow = vx + xr * bx;
   const uint8_t *yrow = vy + p * by;
   const int l = threadIdx.x;
   float sumf = 0.0f;
@@ -169,7 +172,7 @@ __global__ __launch_bounds__(64) void block_dot_pairs(size_t nb, float *s, int32
   }
   if constexpr (!kSums) {
     if (l == 0)
-      s[p] = sumf;
+      s[kGrid ? xr * bs + p : p] = sumf;
   }
 }
 
@@ -546,10 +549,10 @@ int launch_pairs(size_t n, float *s, int32_t *sums, const uint8_t *vx, size_t bx
     return launch_direct_pairs<F>(nb, s, 1, vx, bx, vy, by, npairs, st);
   if (sums)
     tcrv::block_dot_pairs<F, true><<<dim3(static_cast<unsigned>(npairs)), dim3(64), 0, st>>>(
-        nb, s, sums, vx, bx, vy, by);
+        nb, s, sums, vx, bx, vy, by, 0);
   else
     tcrv::block_dot_pairs<F, false><<<dim3(static_cast<unsigned>(npairs)), dim3(64), 0, st>>>(
-        nb, s, sums, vx, bx, vy, by);
+        nb, s, sums, vx, bx, vy, by, 0);
   return launch_status();
 }
 
@@ -600,6 +603,16 @@ int q8_0_rows_direct(size_t nb, float *s, size_t os, const uint8_t *vx, size_t b
 int q4_0_rows_direct(size_t nb, float *s, size_t os, const uint8_t *vx, size_t bx,
                      const uint8_t *vy, size_t by, size_t npairs, void *stream) {
   return rows_direct<DotFmt::kQ4Q8>(nb, s, os, vx, bx, vy, by, npairs, stream);
+}
+
+int q4_0_grid(size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by,
+              size_t nr, size_t nc, size_t bs, void *stream) {
+  if (nr > 65535u || nc > 0x7fffffffu)
+    return TCRV_HIP_ERR_UNSUPPORTED;
+  tcrv::block_dot_pairs<DotFmt::kQ4Q8, false, true>
+      <<<dim3(static_cast<unsigned>(nc), static_cast<unsigned>(nr)), dim3(64), 0,
+         as_stream(stream)>>>(nb, s, nullptr, vx, bx, vy, by, bs);
+  return launch_status();
 }
 
 }  // namespace tcrv_host

@@ -948,6 +948,8 @@ int tcrv_hip_q4_0_q8_0_gemm(size_t n, float *s, const uint8_t *vx, const uint8_t
   }
   const bool rows4 = tcrv_host::aligned4(vx) && tcrv_host::aligned4(vy) &&
                      (nr == 1 || bx % 4 == 0) && by % 4 == 0;
+  if (!(rows4 && nb % 2 == 0) && tcrv_host::q4_0_grid_first(nb, nr, nc))
+    return tcrv_host::q4_0_grid(nb, s, vx, bx, vy, by, nr, nc, bs, stream);
   {
     const int st = tcrv_host::gemm_small(true, rows4, nb, s, vx, bx, vy, by, nr, nc, bs, stream);
     if (st != TCRV_HIP_ERR_UNSUPPORTED)

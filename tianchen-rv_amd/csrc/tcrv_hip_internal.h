@@ -188,6 +188,22 @@ int q8_0_rows_direct(size_t nb, float *s, size_t os, const uint8_t *vx, size_t b
 int q4_0_rows_direct(size_t nb, float *s, size_t os, const uint8_t *vx, size_t bx,
                      const uint8_t *vy, size_t by, size_t npairs, void *stream);
 
+// The Q4_0 x Q8_0 GEMM of few outputs, one wave each (block_dot.hip): any 2-byte aligned rows,
+// any block count.
+int q4_0_grid(size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by,
+              size_t nr, size_t nc, size_t bs, void *stream);
+// Whether it runs a shape of an odd block count or rows off the 4-byte grid before gemm_batch, whose
+// 16 x 16 tiles leave most of the CUs idle there and walk K in a few waves.  Its time by
+// gemm_batch's, medians of 243 such sizes, by outputs (up to 64 / 256 / 512 / 1024 / 2048 / 4096 /
+// 12000): up to 16 blocks 0.96 / 0.97 / 0.97 / 1.00 / 1.02 / 1.23 / 1.8, to 64 0.89 / 0.91 / 0.90 / 0.90 /
+// 0.98 / 1.16 / 1.9, to 128 0.72 / 0.74 / 0.75 / 0.81 / 0.84 / 0.92 / 1.4, to 450 0.69 / 0.76 / 0.76 / 0.82 /
+// 0.83 / 0.93 / 2.0 (us: 135 x 2 x 11552 17.6 -> 10.8, 1097 x 2 x 11936 17.7 -> 14.0; past the bounds
+// 672 x 5 x 8928 12.3 / 13.7, 291 x 5 x 672 3.5 / 3.9).
+inline bool q4_0_grid_first(size_t nb, size_t nr, size_t nc) {
+  const size_t most = nb <= 8 ? 0 : nb <= 16 ? 512 : nb <= 32 ? 1024 : nb <= 64 ? 2048 : 3072;
+  return nr <= most && nc <= most && nr * nc <= most;
+}
+
 // The GEMMs over 16 x 16 tiles with K split over a work-group's waves
 // (gemm_batch.hip): any 2-byte aligned rows, any block count, any nr and nc.
 int gemm_batch(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
