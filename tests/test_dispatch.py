@@ -25,6 +25,7 @@ SIZES = [
     # against the 256-row tiles
     ("q8_0", "plain", 6192, 244, 640, {}, "gemm_wide<false>"),
     ("q4_0", "plain", 977, 1672, 320, {}, "gemm_rows16<true, 4>"),
+    ("q8_0", "plain", 732, 1379, 640, {}, "gemm_rows16<false, 2>"),
     ("q4_0", "plain", 4096, 512, 4160, {}, "gemm_rows16<true, 4>"),
     ("q4_0", "plain", 4096, 1000, 4160, {}, "gemm_wide<true>"),
 ]
@@ -34,3 +35,13 @@ SIZES = [
 def test_kernel_of_a_size(size):
     *call, kw, want = size
     assert launches.kernels([launches.gemm_call(*call, **kw)])[0][-1] == want
+
+
+@pytest.mark.parametrize("quant,nr,nc,n,want", [
+    ("q4_0", 15568, 33, 6656, "pack_tiles_ranges2<true, 2>"),
+    ("q8_0", 4096, 4096, 4096, "pack_tiles_ranges2<false, 2>"),  # 1024 ranges of weights
+    ("q8_0", 4032, 4096, 4096, "pack_tiles_ranges2<false, 1>"),  # 1008
+    ("q8_0", 3001, 4096, 2912, "pack_tiles_ranges2<false, 1>"),
+])
+def test_pack_of_a_workspace_gemm(quant, nr, nc, n, want):
+    assert launches.kernels([launches.gemm_call(quant, "ws", nr, nc, n)])[0][0] == want

@@ -350,15 +350,15 @@ int gemm_rows16(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, cons
 //     138 / 125, 120 x 14581 x 960 Q4_0 19.7 / 17.4);
 //   - else against the 256-row tiles (0.67 / 0.63 a block, few as they may be): four rounds of
 //     64-row work-groups (K 4160, 4096 x 512 61 / 70 against 101 / 93.6, 4096 x 1000 118 / 138
-//     against 101 / 92.5), two of Q8_0 at K under 1024 (6192 x 244 x 640 20.2 / 16.9; Q4_0 977 x
-//     1672 x 320 9.9 / 12.3).
+//     against 101 / 92.5), five of 32-row ones of Q8_0 at K under 1024 (6192 x 244 x 640 17.9 / 16.9,
+//     but 8672 x 116 x 576 13.4 / 15.3; Q4_0 977 x 1672 x 320 9.9 / 12.3).
 bool rows16_first(bool q4, size_t nb, size_t nr, size_t nc, bool few_serves) {
   const size_t w32 = (nr + 31) / 32 * ((nc + 31) / 32), w64 = (nr + 63) / 64 * ((nc + 31) / 32);
   if (few_serves)
     return w32 <= 512 || (w32 <= 768 && (q4 ? nb >= 16 : nb % 16 == 0 && nb <= 48));
   if (nr < 256)
     return q4 ? w64 <= 768 : w32 <= 1280;
-  return nc <= 64 || w64 <= (!q4 && nb < 32 ? 512 : 1024);
+  return nc <= 64 || (!q4 && nb < 32 ? w32 <= 1280 : w64 <= 1024);
 }
 
 int gemm_small(bool q4, bool rows4, size_t nb, float *s, const uint8_t *vx, size_t bx,

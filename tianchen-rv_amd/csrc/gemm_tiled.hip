@@ -342,13 +342,14 @@ struct SpanOperand {
   uint8_t *dst;
 };
 
-template <bool kXQ4>
+template <bool kXQ4, int kXR>
 __global__ __launch_bounds__(256) void pack_tiles_ranges2(size_t nb, SpanOperand x, SpanOperand y) {
-  __shared__ __align__(16) uint8_t raw[kTG * kPackSpan * kQ8Bytes];
-  if (blockIdx.x < x.nranges)
-    pack_range_rows<kXQ4, false, 1>(x.nrows, nb, x.src, x.bx, x.dst, blockIdx.x, x.nranges, raw);
+  __shared__ __align__(16) uint8_t raw[kXR * kTG * kPackSpan * kQ8Bytes];
+  const size_t xgroups = (x.nranges + kXR - 1) / kXR;
+  if (blockIdx.x < xgroups)
+    pack_range_rows<kXQ4, false, kXR>(x.nrows, nb, x.src, x.bx, x.dst, blockIdx.x, x.nranges, raw);
   else
-    pack_range_rows<false, false, 1>(y.nrows, nb, y.src, y.bx, y.dst, blockIdx.x - x.nranges,
+    pack_range_rows<false, false, 1>(y.nrows, nb, y.src, y.bx, y.dst, blockIdx.x - xgroups,
                                      y.nranges, raw);
 }
 
@@ -1619,9 +1620,8 @@ size_t tile_bytes(size_t nrows, size_t nb) {
 
 // Two ranges a work-group where one would make more than three a CU: more bytes in flight a
 // barrier (us, one range against two: 4096 x 4096 Q8_0 6.9 / 6.6, Q4_0 6.5 / 5.8; 11008 x
-// 4096 17.8 / 16.3, 14.7 / 13.0; but 1000 x 4096 3.4 / 3.6, 333 x 4096 2.7 / 3.2).  Not for the
-// two operands of a GEMM, whose records stay in the caches (4096^3 Q8_0: 163 / 167).
-constexpr size_t kPackManyMin = 768;
+// 4096 17.8 / 16.3, 14.7 / 13.0; but 1000 x 4096 3.4 / 3.6, 333 x 4096 2.7 / 3.2).
+constexpr size_t kPackManyMin = 768, kPackPairsMin = 1024;  // one operand; two (pack_tiles_both)
 size_t pack_ranges(size_t nrows, size_t nb) {
   return (nrows + tcrv::kTG - 1) / tcrv::kTG * ((nb + tcrv::kPackSpan - 1) / tcrv::kPackSpan);
 }
@@ -1688,14 +1688,20 @@ int pack_tiles_both(size_t nb, const uint8_t *vx, size_t bx, size_t nr, uint8_t 
   }
   const tcrv::SpanOperand x{vx, bx, nr, pack_ranges(nr, nb), tx};
   const tcrv::SpanOperand y{vy, by, nc, pack_ranges(nc, nb), ty};
-  const size_t grid = x.nranges + y.nranges;
+  // The first operand's ranges in pairs from four a CU, as in the pack of one operand: pack and
+  // GEMM, us, one range against two, 15568 x 33 x 6656 Q4_0 62.9 / 58.7, 13246 x 106 x 6912 Q4_0
+  // 72.6 / 69.2, 14941 x 177 x 3072 Q8_0 48.1 / 45.9; 4096^3 (1024 ranges) Q8_0 163.4 / 162.2; but below
+  // 512 ranges 0.1-0.4 slower.  Kept stores: streamed, 62.1, 84.3 and 52.9 for the first three.
+  const bool pairs = x.nranges >= kPackPairsMin;
+  const size_t grid = (pairs ? (x.nranges + 1) / 2 : x.nranges) + y.nranges;
   if (grid > 0x7fffffffu)
     return TCRV_HIP_ERR_TOO_LARGE;
   const dim3 g(static_cast<unsigned>(grid)), b(256);
-  if (xq4)
-    tcrv::pack_tiles_ranges2<true><<<g, b, 0, st>>>(nb, x, y);
+  auto run = [&](auto kernel) { kernel<<<g, b, 0, st>>>(nb, x, y); };
+  if (pairs)
+    xq4 ? run(tcrv::pack_tiles_ranges2<true, 2>) : run(tcrv::pack_tiles_ranges2<false, 2>);
   else
-    tcrv::pack_tiles_ranges2<false><<<g, b, 0, st>>>(nb, x, y);
+    xq4 ? run(tcrv::pack_tiles_ranges2<true, 1>) : run(tcrv::pack_tiles_ranges2<false, 1>);
   return launch_status();
 }
 
