@@ -45,3 +45,17 @@ def test_kernel_of_a_size(size):
 ])
 def test_pack_of_a_workspace_gemm(quant, nr, nc, n, want):
     assert launches.kernels([launches.gemm_call(quant, "ws", nr, nc, n)])[0][0] == want
+
+
+@pytest.mark.parametrize("quant,rows,nb,bx,want", [
+    ("q8_0", 4037, 11, 11 * 34, "pack_gemm_tiles"),                       # 128 ranges
+    ("q4_0", 1513, 12, 12 * 18, "pack_q4_tiles"),
+    ("q8_0", 4161, 16, 16 * 34 + 2, "pack_tiles_ranges<false, 1, false>"),  # 132, unaligned
+    ("q4_0", 4161, 9, 9 * 18, "pack_tiles_ranges<true, 1, false>"),
+    ("q8_0", 333, 16, 16 * 34, "pack_tiles_ranges<false, 1, true>"),      # few, but whole and aligned
+    ("q8_0", 24577, 9, 9 * 34, "pack_tiles_ranges<false, 2, false>"),
+    ("q4_0", 11008, 128, 128 * 18, "pack_q4_tiles_span"),
+])
+def test_kernel_of_a_pack(quant, rows, nb, bx, want):
+    call = f"tcrv_hip_pack_{quant}_to_gemm_tiles", (rows, nb, launches.X, bx, launches.WS)
+    assert launches.kernels([call]) == [[want]]

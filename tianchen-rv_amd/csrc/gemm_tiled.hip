@@ -286,8 +286,8 @@ __global__ __launch_bounds__(256) void pack_q4_tiles_span(size_t nrows, size_t n
   pack_q4_span(nrows, nb, src, bx, dst, wave, static_cast<int>(threadIdx.x & 63));
 }
 
-// Rows of fewer than 8 blocks: one wave per (group, block) record, lane r = row 64g + r,
-// 16-bit loads.
+// Rows of fewer than 8 blocks, and few rows of others (pack_tiles): one wave per (group, block)
+// record, lane r = row 64g + r, 16-bit loads.
 __global__ __launch_bounds__(256) void pack_gemm_tiles(size_t nrows, size_t nb,
                                                        const uint8_t *src, size_t bx,
                                                        uint8_t *dst, size_t nrec) {
@@ -310,7 +310,7 @@ __global__ __launch_bounds__(256) void pack_gemm_tiles(size_t nrows, size_t nb,
   store_record<false>(dst + rec * kTRec, r, q, d);
 }
 
-// Rows of fewer than 8 blocks: one wave per (group, block) record.
+// Its Q4_0 form.
 __global__ __launch_bounds__(256) void pack_q4_tiles(size_t nrows, size_t nb, const uint8_t *src,
                                                      size_t bx, uint8_t *dst, size_t nrec) {
   const size_t t = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -1622,6 +1622,7 @@ size_t tile_bytes(size_t nrows, size_t nb) {
 // barrier (us, one range against two: 4096 x 4096 Q8_0 6.9 / 6.6, Q4_0 6.5 / 5.8; 11008 x
 // 4096 17.8 / 16.3, 14.7 / 13.0; but 1000 x 4096 3.4 / 3.6, 333 x 4096 2.7 / 3.2).
 constexpr size_t kPackManyMin = 768, kPackPairsMin = 1024;  // one operand; two (pack_tiles_both)
+constexpr size_t kPackRecordsMax = 128;
 size_t pack_ranges(size_t nrows, size_t nb) {
   return (nrows + tcrv::kTG - 1) / tcrv::kTG * ((nb + tcrv::kPackSpan - 1) / tcrv::kPackSpan);
 }
@@ -1630,12 +1631,15 @@ size_t pack_ranges(size_t nrows, size_t nb) {
 int pack_tiles(size_t nrows, size_t nb, const uint8_t *src, size_t bx, uint8_t *dst,
                hipStream_t st, bool q4 = false) {
   using namespace tcrv_host;
-  if (nb >= tcrv::kPackSpan) {
-    const size_t ranges = pack_ranges(nrows, nb);
+  // whole ranges of 16-byte aligned rows
+  const bool whole = nb % tcrv::kPackSpan == 0 && aligned16(src) && bx % 16 == 0;
+  const size_t ranges = pack_ranges(nrows, nb);
+  // Few overlapping or unaligned ranges leave CUs idle where a wave a record does not (us, a wave
+  // a record against ranges: 12 x 1513 rows Q4_0, 48 ranges, 2.20 / 2.37, 42 x 433 Q8_0, 42, 2.18 /
+  // 2.39, 11 x 4037 Q8_0, 128, 2.36 / 2.61; but 107 x 619 Q8_0, 140, 2.96 / 2.68, 364 4.9 / 3.6).
+  if (nb >= tcrv::kPackSpan && (whole || ranges > kPackRecordsMax)) {
     const bool many = ranges >= kPackManyMin;
-    // a Q4_0 wave a range wants whole ranges and 16-byte aligned rows
-    const bool whole = nb % tcrv::kPackSpan == 0 && aligned16(src) && bx % 16 == 0;
-    const bool spans = q4 && many && whole;
+    const bool spans = q4 && many && whole;  // a wave a range
     // A GEMM that follows reads the records: streamed past the caches they cost it more
     // than the pack gains where ranges overlap or rows lie off the lines (pack and GEMM,
     // us, streamed / kept: 1030 x 2537 x 8864 97 / 86, 638 x 371 x 6720 Q4_0 29.3 / 27.6,
