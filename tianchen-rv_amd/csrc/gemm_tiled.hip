@@ -342,15 +342,25 @@ struct SpanOperand {
   uint8_t *dst;
 };
 
+// The first xgrid work-groups pack x: in order, or (group_wgs > 0, the work-groups of a row group)
+// row group g on XCD g % 8, where gemm_tiles32 reads it.
 template <bool kXQ4, int kXR>
-__global__ __launch_bounds__(256) void pack_tiles_ranges2(size_t nb, SpanOperand x, SpanOperand y) {
+__global__ __launch_bounds__(256) void pack_tiles_ranges2(size_t nb, SpanOperand x, SpanOperand y,
+                                                          uint32_t xgrid, uint32_t group_wgs) {
   __shared__ __align__(16) uint8_t raw[kXR * kTG * kPackSpan * kQ8Bytes];
-  const size_t xgroups = (x.nranges + kXR - 1) / kXR;
-  if (blockIdx.x < xgroups)
-    pack_range_rows<kXQ4, false, kXR>(x.nrows, nb, x.src, x.bx, x.dst, blockIdx.x, x.nranges, raw);
-  else
-    pack_range_rows<false, false, 1>(y.nrows, nb, y.src, y.bx, y.dst, blockIdx.x - xgroups,
+  if (blockIdx.x < xgrid) {
+    size_t wg = blockIdx.x;
+    if (group_wgs != 0) {
+      const uint32_t k = blockIdx.x / 8, turn = k / group_wgs;
+      wg = (8 * static_cast<size_t>(turn) + blockIdx.x % 8) * group_wgs + (k - turn * group_wgs);
+      if (wg * kXR >= x.nranges)
+        return;
+    }
+    pack_range_rows<kXQ4, false, kXR>(x.nrows, nb, x.src, x.bx, x.dst, wg, x.nranges, raw);
+  } else {
+    pack_range_rows<false, false, 1>(y.nrows, nb, y.src, y.bx, y.dst, blockIdx.x - xgrid,
                                      y.nranges, raw);
+  }
 }
 
 // ---------------------------------------------------------------- GEMM ---
@@ -1681,10 +1691,10 @@ int pack_tiles(size_t nrows, size_t nb, const uint8_t *src, size_t bx, uint8_t *
 }
 
 // Both operands of a GEMM (xq4: the weights vx are Q4_0): one launch from 8 blocks a row,
-// else one per operand.
+// else one per operand.  by_xcd: the weights' row groups go round the XCDs.
 int pack_tiles_both(size_t nb, const uint8_t *vx, size_t bx, size_t nr, uint8_t *tx,
                     const uint8_t *vy, size_t by, size_t nc, uint8_t *ty, hipStream_t st,
-                    bool xq4 = false) {
+                    bool xq4, bool by_xcd) {
   using namespace tcrv_host;
   if (nb < tcrv::kPackSpan) {
     const int rc = pack_tiles(nr, nb, vx, bx, tx, st, xq4);
@@ -1697,11 +1707,19 @@ int pack_tiles_both(size_t nb, const uint8_t *vx, size_t bx, size_t nr, uint8_t 
   // 72.6 / 69.2, 14941 x 177 x 3072 Q8_0 48.1 / 45.9; 4096^3 (1024 ranges) Q8_0 163.4 / 162.2; but below
   // 512 ranges 0.1-0.4 slower.  Kept stores: streamed, 62.1, 84.3 and 52.9 for the first three.
   const bool pairs = x.nranges >= kPackPairsMin;
-  const size_t grid = (pairs ? (x.nranges + 1) / 2 : x.nranges) + y.nranges;
+  const size_t groups = (nr + tcrv::kTG - 1) / tcrv::kTG, each = x.nranges / groups;
+  const size_t group_wgs = !by_xcd ? 0 : !pairs ? each : each % 2 == 0 ? each / 2 : 0;
+  const size_t xgrid = group_wgs != 0 ? (groups + 7) / 8 * 8 * group_wgs
+                       : pairs        ? (x.nranges + 1) / 2
+                                      : x.nranges;
+  const size_t grid = xgrid + y.nranges;
   if (grid > 0x7fffffffu)
     return TCRV_HIP_ERR_TOO_LARGE;
   const dim3 g(static_cast<unsigned>(grid)), b(256);
-  auto run = [&](auto kernel) { kernel<<<g, b, 0, st>>>(nb, x, y); };
+  auto run = [&](auto kernel) {
+    kernel<<<g, b, 0, st>>>(nb, x, y, static_cast<uint32_t>(xgrid),
+                            static_cast<uint32_t>(group_wgs));
+  };
   if (pairs)
     xq4 ? run(tcrv::pack_tiles_ranges2<true, 2>) : run(tcrv::pack_tiles_ranges2<false, 2>);
   else
@@ -1897,6 +1915,17 @@ bool ws_rows_few_first(size_t nb, const uint8_t *vx, size_t bx, const uint8_t *v
          !tiles16_first(nr, nc) && tiles64_of(nr, nc) <= 448;
 }
 
+// Whether the workspace entries pack weight row group g on XCD g % 8: gemm_tiles32, whose tile rows
+// are the groups, reads it there unless its work-groups divide by 8 (tile_of then deals them in
+// runs), and finds in that XCD's L2 what fits the eight of them (pack and GEMM, us, in order
+// against this: 13637 x 166 x 1024 Q4_0 24.4 / 20.2, 8193 x 196 x 1024 Q8_0 18.7 / 16.4).  From 64 groups,
+// for an even spread.
+bool pack_by_xcd(size_t nb, size_t nr, size_t nc) {
+  const size_t tiles64 = tiles64_of(nr, nc);
+  return tiles32_first(tiles128_of(nr, nc), tiles64, nb) && !tiles16_first(nr, nc) &&
+         tiles64 % 8 != 0 && nr > 63 * static_cast<size_t>(tcrv::kTG);
+}
+
 // Shapes that take a workspace by the rule below but do not need it: few outputs,
 // where gemm_batch and gemm_rows16 read the plain rows faster than they are packed (us, K
 // 4096, Q4_0 / Q8_0, against pack and tiles: 4096 x 32 10.0 / 11.0 against 27 / 24,
@@ -1960,7 +1989,8 @@ int tcrv_hip_q8_0_q8_0_gemm_ws(size_t n, float *s, const uint8_t *vx, const uint
   uint8_t *tx = static_cast<uint8_t *>(workspace);
   uint8_t *ty = tx + tx_bytes;  // tx_bytes is a multiple of 2176 = 16 * 136
   hipStream_t st = as_stream(stream);
-  const int rc = pack_tiles_both(nb, vx, bx, nr, tx, vy, by, nc, ty, st);
+  const int rc = pack_tiles_both(nb, vx, bx, nr, tx, vy, by, nc, ty, st, false,
+                                 pack_by_xcd(nb, nr, nc));
   if (rc != TCRV_HIP_OK)
     return rc;
   return gemm_tiles(nb, s, tx, ty, nr, nc, bs, st);
@@ -2028,7 +2058,8 @@ int tcrv_hip_q4_0_q8_0_gemm_ws(size_t n, float *s, const uint8_t *vx, const uint
   uint8_t *tx = static_cast<uint8_t *>(workspace);
   uint8_t *ty = tx + tx_bytes;  // tx_bytes is a multiple of 2176 = 16 * 136
   hipStream_t st = as_stream(stream);
-  const int rc = pack_tiles_both(nb, vx, bx, nr, tx, vy, by, nc, ty, st, true);
+  const int rc = pack_tiles_both(nb, vx, bx, nr, tx, vy, by, nc, ty, st, true,
+                                 pack_by_xcd(nb, nr, nc));
   if (rc != TCRV_HIP_OK)
     return rc;
   return gemm_tiles(nb, s, tx, ty, nr, nc, bs, st, true);
