@@ -14,10 +14,13 @@ SIZES = [
     ("q8_0", "plain", 4096, 64, 4096, {}, "gemm_rows16<false, 2>"),
     # few outputs, where gemm_rows_few serves
     ("q4_0", "plain", 4096, 192, 4096, {}, "gemm_rows16<true, 2>"),
-    ("q8_0", "plain", 4096, 192, 4096, {}, "gemm_rows_few<false>"),
+    ("q8_0", "plain", 4096, 192, 4096, {}, "gemm_rows16<false, 2>"),
+    ("q8_0", "plain", 4096, 192, 4352, {}, "gemm_rows_few<false>"),
     ("q8_0", "plain", 6457, 75, 512, {}, "gemm_rows16<false, 2>"),
     ("q8_0", "plain", 4894, 127, 256, {}, "gemm_rows_few<false>"),
     ("q4_0", "plain", 1166, 596, 256, {}, "gemm_rows_few<true>"),
+    ("q8_0", "plain", 18006, 21, 1792, {}, "gemm_rows16<false, 2>"),
+    ("q4_0", "plain", 790, 1238, 3584, {}, "gemm_rows16<true, 4>"),
     # few weight rows and many tokens, K no multiple of 256
     ("q8_0", "plain", 190, 8881, 10432, {}, "gemm_occ<false>"),
     ("q4_0", "plain", 120, 14581, 960, {}, "gemm_occ<true>"),

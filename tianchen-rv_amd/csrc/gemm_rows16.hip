@@ -341,10 +341,12 @@ int gemm_rows16(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, cons
 
 // Whether gemm_rows16 runs a shape of 4-byte aligned rows.  Measured over the same sizes, us:
 //   - against gemm_rows_few, where that serves: up to two rounds of 32-row work-groups (4096 x 128
-//     x 4096 18.4 / 16.6 against 31.0 / 26.7), and three of Q4_0 (0.193 against 0.214 a block) but
-//     for K 256, half a chunk (1166 x 596 5.8 / 5.0); three of Q8_0 cost as much (0.193 against 0.179)
-//     but for few whole chunks (6457 x 75 x 512 5.5 / 6.1, 2659 x 258 x 1536 11.5 / 12.2, but
-//     4894 x 127 x 256 5.2 / 4.7, 107 x 4937 x 1792 14.6 / 13.5);
+//     x 4096 18.4 / 16.6 against 31.0 / 26.7), four where its 64 x 64 ones, half empty at few tokens,
+//     take two (18006 x 21 x 1792 Q8_0 13.7 / 18.9, 790 x 1238 x 3584 Q4_0 27.9 / 34.6), and three of
+//     Q4_0 (0.193 against 0.214 a block) but for K 256, half a chunk (1166 x 596 5.8 / 5.0); three
+//     of Q8_0 with K of whole chunks, a part chunk costing nearly a whole one (150 sizes, by
+//     gemm_rows_few's time: 16 blocks 0.90, 64 0.93, 128 and 320 0.97, but 8 blocks 1.15, 24 1.08, 40
+//     1.04, 72 1.02; 4245 x 142 x 2048 13.5 / 14.8 us);
 //   - else, under 256 weight rows, against the 128 x 128 tiles (one round 0.40 / 0.36 a block): three
 //     rounds of 64-row work-groups (Q4_0), five of 32-row ones (Q8_0) (190 x 8881 x 10432 Q8_0
 //     138 / 125, 120 x 14581 x 960 Q4_0 19.7 / 17.4);
@@ -354,8 +356,11 @@ int gemm_rows16(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, cons
 //     but 8672 x 116 x 576 13.4 / 15.3; Q4_0 977 x 1672 x 320 9.9 / 12.3).
 bool rows16_first(bool q4, size_t nb, size_t nr, size_t nc, bool few_serves) {
   const size_t w32 = (nr + 31) / 32 * ((nc + 31) / 32), w64 = (nr + 63) / 64 * ((nc + 31) / 32);
-  if (few_serves)
-    return w32 <= 512 || (w32 <= 768 && (q4 ? nb >= 16 : nb % 16 == 0 && nb <= 48));
+  if (few_serves) {
+    if (w32 <= 512 || (nr + 63) / 64 * ((nc + 63) / 64) > 256)
+      return w32 <= 1024;
+    return w32 <= 768 && (q4 ? nb >= 16 : nb % 16 == 0);
+  }
   if (nr < 256)
     return q4 ? w64 <= 768 : w32 <= 1280;
   return nc <= 64 || (!q4 && nb < 32 ? w32 <= 1280 : w64 <= 1024);
