@@ -19,11 +19,14 @@ SIZES = [
     (27, 19, 11, 0, 0, 0, BATCH8),     # 513
     (127, 8, 31, 0, 6, 0, GRID),
     (33, 31, 33, 0, 0, 0, GRID),
-    (64, 48, 128, 2, 2, 0, GRID),      # one whole chunk, 3072 outputs
-    (77, 40, 128, 2, 2, 0, BATCH16),   # 3080
+    (64, 32, 128, 2, 2, 0, GRID),      # one whole chunk, 2048 outputs
+    (64, 33, 128, 2, 2, 0, BATCH16),   # 2112, 176 a tile
+    (832, 4, 129, 0, 0, 0, GRID),      # 3328, 64 a tile
+    (1665, 2, 129, 0, 0, 0, BATCH8),
+    (560, 5, 129, 0, 0, 0, BATCH8),    # 2800, 80 a tile
     (5, 3, 257, 0, 4, 2, GRID),        # a chunk of one block
     (200, 20, 131, 0, 0, 2, BATCH8),   # three 8-wave chunks, the last of three blocks
-    (1600, 2, 257, 0, 4, 0, BATCH8),   # five chunks, one block in the last
+    (1700, 2, 257, 0, 4, 0, BATCH8),   # five chunks, one block in the last
     (520, 7, 65, 0, 0, 0, BATCH16),    # 16 waves, nine of them with blocks
     (400, 7, 63, 2, 6, 2, BATCH8),     # every slice, the last one block short
     (2, 2, 8, 2, 2, 0, BATCH8),
@@ -37,7 +40,9 @@ def test_rule(nr, nc, nb, xpad, ypad, off, kernel):
     assert launches.kernels([call]) == [[kernel]]
 
 
-@pytest.mark.parametrize("nr,nc,n", [(135, 2, 11552), (1097, 2, 11936), (1, 1621, 2720)])
+@pytest.mark.parametrize("nr,nc,n", [(135, 2, 11552), (1097, 2, 11936), (1, 1621, 2720),
+                                      (2, 1623, 3936), (1502, 2, 9504),
+                                      (517, 4, 2336)])
 def test_shapes_that_gemm_batch_is_slower_at(nr, nc, n):
     assert launches.kernels([launches.gemm_call("q4_0", "plain", nr, nc, n)]) == [[GRID]]
 

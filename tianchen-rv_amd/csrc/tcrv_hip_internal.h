@@ -198,10 +198,13 @@ int q4_0_grid(size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *
 // 12000): up to 16 blocks 0.96 / 0.97 / 0.97 / 1.00 / 1.02 / 1.23 / 1.8, to 64 0.89 / 0.91 / 0.90 / 0.90 /
 // 0.98 / 1.16 / 1.9, to 128 0.72 / 0.74 / 0.75 / 0.81 / 0.84 / 0.92 / 1.4, to 450 0.69 / 0.76 / 0.76 / 0.82 /
 // 0.83 / 0.93 / 2.0 (us: 135 x 2 x 11552 17.6 -> 10.8, 1097 x 2 x 11936 17.7 -> 14.0; past the bounds
-// 672 x 5 x 8928 12.3 / 13.7, 291 x 5 x 672 3.5 / 3.9).
+// 672 x 5 x 8928 12.3 / 13.7, 291 x 5 x 672 3.5 / 3.9).  Past 2048 outputs where gemm_batch's tiles hold
+// few of them (1502 x 2 x 9504 15.0 -> 13.0, but 7 x 413 x 8768 11.9 / 15.5).
 inline bool q4_0_grid_first(size_t nb, size_t nr, size_t nc) {
-  const size_t most = nb <= 8 ? 0 : nb <= 16 ? 512 : nb <= 32 ? 1024 : nb <= 64 ? 2048 : 3072;
-  return nr <= most && nc <= most && nr * nc <= most;
+  const size_t most = nb <= 8 ? 0 : nb <= 16 ? 512 : nb <= 32 ? 1024 : nb <= 64 ? 2048 : 3328;
+  if (nr > most || nc > most || nr * nc > most)
+    return false;
+  return nr * nc <= 2048 || nr * nc <= 64 * ((nr + 15) / 16) * ((nc + 15) / 16);
 }
 
 // The GEMMs over 16 x 16 tiles with K split over a work-group's waves
