@@ -32,7 +32,7 @@ KERNELS = {
     "gemv_q4_0_q8_0": "gemv_q4_0_q8_0_direct",
     "q8_0_q8_0_gemm": "gemm_wide<false>",
     "q8_0_q8_0_gemm_tiles": "gemm_tiles256_q8",
-    "pack_both_to_gemm_tiles": "pack_gemm_tiles_span2",
+    "pack_both_to_gemm_tiles": "pack_tiles_ranges2",
     "calib": "add_f32_vec4",
 }
 CALIB_BYTES = {"FETCH_SIZE": 8 << 24, "WRITE_SIZE": 4 << 24}  # per add_f32 launch, n = 2^24
