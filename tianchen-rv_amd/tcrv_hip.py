@@ -177,6 +177,17 @@ def _raw_stream_getter():
 _raw_stream = None
 
 
+def _forget_raw_stream():
+    """A forked child asks torch anew, which refuses a device that the parent initialised; the
+    raw getters do not look."""
+    global _raw_stream
+    _raw_stream = None
+
+
+if hasattr(os, "register_at_fork"):
+    os.register_at_fork(after_in_child=_forget_raw_stream)
+
+
 def _stream(stream) -> int:
     global _raw_stream
     if stream is None:
