@@ -218,7 +218,8 @@ TCRV_HIP_API int tcrv_hip_gemv_q4_0_q8_0(size_t n, float *s, const uint8_t *vx, 
  * bit-identical for every value.  For n = 2048 and 1024, 4 selects the
  * lane-group kernels, whose waves own 4 or 8 rows by n and nr.  Shapes served
  * by the LDS-staged kernel (odd n/32, rows not 4-byte aligned) ignore it, and the plain
- * entry runs some longer rows on gemv_long.  Any other value returns TCRV_HIP_ERR_BAD_SIZE. */
+ * entry runs up to 2048 weight rows of 130 to 512 blocks on gemv_long, which this one does not.
+ * Any other value returns TCRV_HIP_ERR_BAD_SIZE. */
 TCRV_HIP_API int tcrv_hip_gemv_q4_0_q8_0_shaped(size_t n, float *s, const uint8_t *vx, size_t bx,
                                                 const uint8_t *vy, size_t nr, int rows_per_wave,
                                                 void *stream);
@@ -255,10 +256,14 @@ TCRV_HIP_API int tcrv_hip_q8_0_q8_0_gemm_tiles(size_t n, float *s, const uint8_t
                                                const uint8_t *ty, size_t nr, size_t nc,
                                                size_t bs, void *stream);
 /* tcrv_hip_q8_0_q8_0_gemm (same ABI and results) with a caller-owned device
- * workspace: both operands are packed into it (tx then ty) and the tiled GEMM
- * runs.  Needs tcrv_hip_q8_0_q8_0_gemm_workspace_bytes(n, nr, nc) bytes, 16-byte
- * aligned; shapes the tiled kernel does not serve (nr < 256, nc < 2, n/32 over
- * 1 973 789) run tcrv_hip_q8_0_q8_0_gemm and leave the workspace untouched.
+ * workspace of tcrv_hip_q8_0_q8_0_gemm_workspace_bytes(n, nr, nc) bytes, 16-byte
+ * aligned, for the kernels that run on packed operands.  What it holds after a
+ * call is unspecified: few outputs run from the plain rows and do not write it,
+ * though it is required and checked all the same.  It is neither required nor
+ * looked at for nr < 256, nc < 2, n < 32 or n/32 over 1 973 789; up to 24 tokens
+ * over an even n/32 and 4-byte aligned rows and strides; and with 16-byte aligned
+ * rows and strides and n a multiple of 256 up to 4096, for 257 and more 32 x 32
+ * output tiles in at most 448 of 64 x 64.
  * Calls that share a workspace must be ordered (one stream). */
 TCRV_HIP_API size_t tcrv_hip_q8_0_q8_0_gemm_workspace_bytes(size_t n, size_t nr, size_t nc);
 TCRV_HIP_API int tcrv_hip_q8_0_q8_0_gemm_ws(size_t n, float *s, const uint8_t *vx,
@@ -298,11 +303,8 @@ TCRV_HIP_API int tcrv_hip_q4_0_q8_0_gemm_tiles(size_t n, float *s, const uint8_t
                                                const uint8_t *ty, size_t nr, size_t nc,
                                                size_t bs, void *stream);
 /* tcrv_hip_q4_0_q8_0_gemm (same ABI and results) with a caller-owned device
- * workspace: the Q4_0 weights and the Q8_0 tokens are packed into it (tx then
- * ty, one launch) and the tiled GEMM runs.  Needs
- * tcrv_hip_q4_0_q8_0_gemm_workspace_bytes(n, nr, nc) bytes, 16-byte aligned;
- * shapes the tiled kernel does not serve (nr < 256, nc < 2, n/32 over
- * 1 973 789) run tcrv_hip_q4_0_q8_0_gemm and leave the workspace untouched.
+ * workspace of tcrv_hip_q4_0_q8_0_gemm_workspace_bytes(n, nr, nc) bytes, required,
+ * looked at and written (or not) as tcrv_hip_q8_0_q8_0_gemm_ws's.
  * Calls that share a workspace must be ordered (one stream). */
 TCRV_HIP_API size_t tcrv_hip_q4_0_q8_0_gemm_workspace_bytes(size_t n, size_t nr, size_t nc);
 TCRV_HIP_API int tcrv_hip_q4_0_q8_0_gemm_ws(size_t n, float *s, const uint8_t *vx,

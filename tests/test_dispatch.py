@@ -1,8 +1,11 @@
 """Which kernel an entry runs at a size: the shipped rules, replayed without a GPU
 (tests/launches.py)."""
+import random
+
 import pytest
 
 import launches
+import tcrv_hip
 
 # quant, entry, weight rows, tokens, n, keyword arguments of gemm_call, kernel
 SIZES = [
@@ -62,3 +65,42 @@ def test_pack_of_a_workspace_gemm(quant, nr, nc, n, want):
 def test_kernel_of_a_pack(quant, rows, nb, bx, want):
     call = f"tcrv_hip_pack_{quant}_to_gemm_tiles", (rows, nb, launches.X, bx, launches.WS)
     assert launches.kernels([call]) == [[want]]
+
+
+def workspace_needed(quant, nr, nc, n, xpad, ypad):
+    """What include/tcrv_hip.h says of the workspace entries."""
+    nb = n // 32
+    bx, by = nb * (18 if quant == "q4_0" else 34) + xpad, nb * 34 + ypad
+
+    def aligned(k):
+        return bx % k == 0 and by % k == 0
+
+    def tiles(k):
+        return -(-nr // k) * -(-nc // k)
+
+    if nr < 256 or nc < 2 or nb < 1:
+        return False
+    if nc <= 24 and nb % 2 == 0 and aligned(4):
+        return False
+    return not (nb % 8 == 0 and nb <= 128 and aligned(16) and tiles(32) > 256 and tiles(64) <= 448)
+
+
+@pytest.mark.parametrize("quant", ["q4_0", "q8_0"])
+def test_workspace_is_required_where_the_header_says(quant):
+    """A missing workspace is refused exactly there, and nothing is launched; elsewhere the call
+    runs.  What a call writes into it is unspecified (few outputs: nothing)."""
+    rng = random.Random(5)
+    sizes = [(255, 64, 4096, 0, 0), (256, 1, 4096, 0, 0), (256, 2, 32, 0, 0), (256, 24, 4096, 0, 0),
+             (256, 25, 4096, 0, 0), (256, 24, 4096 + 32, 0, 0), (256, 24, 4096, 2, 0),
+             (4096, 128, 4096, 0, 0), (4096, 128, 4352, 0, 0), (4096, 128, 4096, 4, 0),
+             (4096, 448, 4096, 0, 0), (4096, 449, 4096, 0, 0), (512, 512, 4096, 0, 0),
+             (512, 544, 4096, 0, 0)]
+    sizes += [(rng.randint(200, 6000), rng.randint(1, 600), 32 * rng.randint(1, 140),
+               rng.choice((0, 0, 2, 4, 16)), rng.choice((0, 0, 2, 16))) for _ in range(200)]
+    calls = []
+    for nr, nc, n, xpad, ypad in sizes:
+        name, args = launches.gemm_call(quant, "ws", nr, nc, n, xpad, ypad)
+        calls.append((name, args[:-2] + (0, 0)))
+    for size, (status, xs) in zip(sizes, launches.replay(calls)):
+        want = tcrv_hip.ERR_NULL_POINTER if workspace_needed(quant, *size) else 0
+        assert status == want and bool(xs) == (want == 0), (size, status, xs)

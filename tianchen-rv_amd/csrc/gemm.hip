@@ -11,7 +11,8 @@
 // fold of that block is applied to the tile right away, in ascending block
 // order, so every output element sees the reference's sequence of roundings.
 //
-// Two kernels, for rows that are 4-byte aligned (others run gemm_batch.hip):
+// Two kernels, for rows that are 4-byte aligned (others run gemm_rows16.hip and
+// gemm_batch.hip, as do fewer outputs):
 //   gemm_wide<false>  at least 256 weight rows: 256 x 128 output tile per
 //                     work-group (the fast path, below);
 //   gemm_occ<false>   fewer weight rows: 128 x 128.

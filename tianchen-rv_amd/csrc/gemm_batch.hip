@@ -28,8 +28,9 @@
 // counts a kernel of one wave an output or the raw 128 x 128 tiles):
 //   8 tokens Q4_0 7.8 -> 6.2, Q8_0 8.8 -> 7.0; 16 tokens 15.4 -> 6.2, 15.8 ->
 //   7.0; 32 tokens 30.6 -> 10.0, 26.4 -> 11.0; 3001 x 6 x 2912 (91 blocks)
-//   27.5 -> 7.0, 397 -> 7.5; one token, 4096 x 14304 (447 blocks) 26.2 -> 19.3,
-//   2110 -> 21.
+//   27.5 -> 7.0, 397 -> 7.5; one token, Q8_0 4096 x 14304 (447 blocks) 2110 -> 21
+//   (Q4_0 decodes on gemv.hip's LDS-staged kernel, and its few outputs of odd block
+//   counts a wave each, block_dot.hip).
 #include "tcrv_hip_internal.h"
 #include "mfma_fold.h"
 #include "tile_order.h"

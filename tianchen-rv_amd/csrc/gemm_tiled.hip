@@ -1,10 +1,12 @@
 // gemm_tiled.hip -- the a9 Q8_0 x Q8_0 and a7 Q4_0 x Q8_0 GEMMs over operands
 // in the GEMM-tile layout, staged into LDS by DMA (buffer_load_dwordx4 ... lds,
 // global_load_lds_dwordx4): no staging registers and no staging VALU, so every
-// VGPR and VALU cycle goes to the fold.  Two work-group tiles: 256 weight rows
-// x 128 tokens (16 waves of 2 tiles, gemm_tiles_q8 / gemm_tiles_q4) and 256 x
-// 256 (8 waves of 2 x 4 tiles, gemm_tiles256_q8 / gemm_tiles256_q4); the
-// entries pick per shape (tiles256_first), the results are the same bits.
+// VGPR and VALU cycle goes to the fold.  Three work-group tiles: 256 weight rows
+// x 128 tokens (16 waves of 2 tiles, gemm_tiles_q8 / gemm_tiles_q4), 256 x 256
+// and 192 x 256 (8 waves of 2 x 4 or 3 x 2 tiles, gemm_tiles256_q8 /
+// gemm_tiles256_q4), picked per shape by rounds (tile_shape); where even 256 x 128
+// would leave CUs idle one 32 x 32 or 16 x 16 tile a wave without LDS (gemm_tiles32,
+// gemm_tiles16).  The results are the same bits.
 //
 // GEMM-tile layout of a Q8_0 matrix of nrows rows x nb blocks (the same bytes
 // as the plain rows, regrouped): rows in groups of 64; for group g and block b

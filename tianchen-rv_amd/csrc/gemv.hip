@@ -5,8 +5,11 @@
 // row ir and activation column col (RVVToEmitCBlockQuantLinear.cpp:1691-2121;
 // RVVOps.td:4147-4151).  The decode GEMV kernel below keeps that per-element
 // definition and its fold order, fma(fl((float)sumi*d_x), d_y, sumf) in
-// ascending block order; with more tokens, rows that are not 4-byte aligned and odd
-// block counts run gemm_batch.hip.
+// ascending block order, for rows of any 2-byte alignment and any block count, and the
+// multi-column form does for two to four tokens over an even block count and 4-byte aligned
+// rows.  Other GEMM calls run block_dot.hip's wave an output (few outputs), gemm_batch.hip,
+// gemm_rows16.hip, gemm_tiled.hip's gemm_rows_few or gemm.hip, by the rules at their
+// declarations.
 #include "tcrv_hip_internal.h"
 
 namespace tcrv {

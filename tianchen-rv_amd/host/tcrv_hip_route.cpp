@@ -255,6 +255,16 @@ const tcrv_hip_schedule kSchedules[] = {
     {"tcrv_rvv.q4_0_q8_0_gemm", TCRV_HIP_M_PREFILL, "gemm_tiles256_q4", "work_group_tokens", 256,
      1, nullptr, -1.0,
      "8 waves of 2 x 4 transposed tiles, a token tile's d_y read once for both weight tiles"},
+    // the tiled GEMMs of 256 tokens: weight rows per work-group tile
+    {"tcrv_rvv.q8_0_q8_0_gemm", TCRV_HIP_M_PREFILL, "gemm_tiles256_q8", "work_group_rows", 192, 0,
+     nullptr, -1.0,
+     "8 waves of 3 x 2 32x32 tiles; where it takes fewer rounds' time (11008 x 1000: one round)"},
+    {"tcrv_rvv.q8_0_q8_0_gemm", TCRV_HIP_M_PREFILL, "gemm_tiles256_q8", "work_group_rows", 256, 1,
+     nullptr, -1.0, "8 waves of 2 x 4 32x32 tiles; the 4096^3 reference shape is one round"},
+    {"tcrv_rvv.q4_0_q8_0_gemm", TCRV_HIP_M_PREFILL, "gemm_tiles256_q4", "work_group_rows", 192, 0,
+     nullptr, -1.0, "8 waves of 3 x 2 transposed tiles; where it takes fewer rounds' time"},
+    {"tcrv_rvv.q4_0_q8_0_gemm", TCRV_HIP_M_PREFILL, "gemm_tiles256_q4", "work_group_rows", 256, 1,
+     nullptr, -1.0, "8 waves of 2 x 4 transposed tiles; the 4096^3 reference shape is one round"},
     // the 256 x 128 tiled Q8_0 GEMM: blocks per K chunk (two LDS stages for
     // 5-6 blocks, three for 3-4; the 256 x 256 kernel fits two stages of 4);
     // a build-time constant
