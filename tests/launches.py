@@ -12,6 +12,7 @@ import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
+LIB = os.path.join(ROOT, "tianchen-rv_amd", "libtcrv_hip.so")
 
 # Device addresses of the replayed calls: never read, only their alignment counts.
 S, X, Y, WS = 1 << 40, 2 << 40, 3 << 40, 4 << 40
