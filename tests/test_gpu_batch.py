@@ -1,6 +1,7 @@
 """The 16 x 16-tile GEMM that splits K over a work-group's waves (gemm_batch.hip),
 through the plain GEMM, GEMV and workspace entries, against the oracle bit for bit:
-few tokens, and rows that are only 2-byte aligned at any number of tokens."""
+few tokens, and rows that are only 2-byte aligned at any number of tokens (Q4_0 runs a few of
+these sizes a wave an output; its own past that rule are in test_gpu_grid.py)."""
 import numpy as np
 import pytest
 import torch

@@ -203,9 +203,8 @@ def test_gemm_tiled_operands_over_2_gib(hip, oracle, dev):
 @pytest.mark.parametrize("nb", [1973789, 1973790])
 def test_q8_0_gemm_ws_at_the_tiled_block_bound(hip, oracle, dev, nb):
     """K at the workspace entry's bound (the 256-row tiled kernels' 32-bit DMA chunk offset):
-    n/32 = 1 973 789 blocks (odd: no multi-column GEMV) is packed and runs the tiled kernel of
-    this shape -- one 32 x 32 tile a wave, its last block's records 2 KB below 2^32 bytes into
-    a group; one block more runs the plain GEMM.  256 weight rows x 2 tokens; every row repeats
+    n/32 = 1 973 789 blocks takes and checks a workspace, one block more does not; both run
+    gemm_batch at these few outputs (packed operands of that K: the test below).  256 weight rows x 2 tokens; every row repeats
     a 2048-block pattern along K (built on the device), so the sampled rows' bytes are known on
     the host."""
     nr, nc, pat = 256, 2, 2048
@@ -228,3 +227,32 @@ def test_q8_0_gemm_ws_at_the_tiled_block_bound(hip, oracle, dev, nb):
     a_rows = np.ascontiguousarray(np.tile(base_a, (1, reps))[:, :rb])
     want = oracle.gemm_q8_0(n, w_rows, a_rows, rb, len(pick), nc, rb, nc, 8).reshape(len(pick), nc)
     assert_f32_parity(got[pick], want, what=f"q8_0 gemm_ws at nb = {nb}")
+
+
+def test_q8_0_gemm_tiles_at_the_block_bound(hip, oracle, dev):
+    """Packed operands with the last block's records 2 KB below 2^32 bytes into a row group: the
+    pack and the one-tile-a-wave kernel.  65 weight rows (a second group of one) x 2 tokens; one
+    block more is refused."""
+    nr, nc, nb, pat = 65, 2, 1973789, 2048
+    n, rb, reps = nb * 32, nb * 34, -(-nb // pat)
+    base_w = synth.q8_0_matrix(nr, pat * 32, 1033, 0.02)
+    base_a = synth.q8_0_matrix(nc, pat * 32, 1034, 1.0)
+    dw = torch.from_numpy(base_w).to(dev).repeat(1, reps)[:, :rb].contiguous()
+    da = torch.from_numpy(base_a).to(dev).repeat(1, reps)[:, :rb].contiguous()
+    tx = torch.empty(hip.gemm_tiles_bytes(nr, nb), dtype=torch.uint8, device=dev)
+    ty = torch.empty(hip.gemm_tiles_bytes(nc, nb), dtype=torch.uint8, device=dev)
+    s = torch.full((nr * nc,), float("nan"), dtype=torch.float32, device=dev)
+    hip.pack_q8_0_to_gemm_tiles(nr, nb, dw, rb, tx)
+    hip.pack_q8_0_to_gemm_tiles(nc, nb, da, rb, ty)
+    hip.q8_0_q8_0_gemm_tiles(n, s, tx, ty, nr, nc, nc)
+    got = s.view(nr, nc).cpu().numpy()
+    with pytest.raises(hip.TcrvHipError) as e:
+        hip.q8_0_q8_0_gemm_tiles(n + 32, s, tx, ty, nr, nc, nc)
+    assert e.value.status == hip.ERR_TOO_LARGE
+    del dw, da, tx, ty, s
+    free()
+    pick = np.array([0, 31, 64])
+    w_rows = np.ascontiguousarray(np.tile(base_w[pick], (1, reps))[:, :rb])
+    a_rows = np.ascontiguousarray(np.tile(base_a, (1, reps))[:, :rb])
+    want = oracle.gemm_q8_0(n, w_rows, a_rows, rb, len(pick), nc, rb, nc, 8).reshape(len(pick), nc)
+    assert_f32_parity(got[pick], want, what="q8_0 gemm_tiles at the block bound")

@@ -1,4 +1,5 @@
-"""The GEMM-tile packs by 8-block ranges (gemm_tiled.hip) against the documented layout byte for
+"""The GEMM-tile packs (gemm_tiled.hip; up to 128 ragged or unaligned ranges by records, the others by
+8-block ranges) against the documented layout byte for
 byte: the last range short by 1 to 7 blocks, rows at 2-byte alignment, one and two ranges a
 work-group with an odd number of ranges, and the Q4_0 wave a range of many aligned rows."""
 import numpy as np

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+import launches
 import synth
 from gpu_util import assert_f32_parity, assert_f32_parity_nan, empty_dev, from_dev, q4_tiles_gemm, to_dev
 
@@ -365,16 +366,16 @@ def test_q4_0_gemm_multi_column(hip, oracle, dev, nr, nc, nb):
 @pytest.mark.parametrize("nr,nc,nb,ypad", [
     (4096, 2, 128, 0),   # one chunk, two columns
     (4096, 3, 128, 0),   # a four-column group with three present
-    (100, 7, 130, 16),   # partial work-group, two chunks (the second of 2 blocks), 4 + 3
-    (300, 6, 258, 4),    # three chunks, 4 + 2 columns
-    (64, 9, 64, 0),      # nb < 128, 4 + 4 + 1 (the last column through the GEMV)
-    (48, 64, 8, 0),      # the largest token count of the multi-column path
-    (40, 5, 7, 0),       # odd nb: the MFMA GEMM instead
+    (100, 7, 130, 16),   # 130 blocks: a chunk of two after whole ones
+    (300, 6, 258, 4),
+    (64, 9, 64, 0),
+    (48, 64, 8, 0),
+    (40, 5, 7, 0),       # odd nb
 ])
 def test_q4_0_gemm_few_tokens(hip, oracle, dev, nr, nc, nb, ypad):
-    """The a7 GEMM with a few tokens (batched decode) runs as GEMVs over groups
-    of up to four activation columns, the weights read once per group: every
-    output equals the oracle's, and the output row padding stays untouched."""
+    """The a7 GEMM with a few tokens (batched decode; two to four as one multi-column GEMV, more on
+    16 x 16 MFMA tiles): every output equals the oracle's, and the output row padding stays
+    untouched."""
     n = nb * 32
     w = synth.q4_0_matrix(nr, n, 1017, 0.02)
     a = np.pad(synth.q8_0_matrix(nc, n, 1016, 1.0), ((0, 0), (0, ypad)))
@@ -392,17 +393,17 @@ def test_q4_0_gemm_few_tokens(hip, oracle, dev, nr, nc, nb, ypad):
 
 @pytest.mark.parametrize("nr,nc,nb,ypad", [
     (4096, 2, 128, 0),   # one chunk, two columns
-    (4096, 5, 128, 0),   # an eight-column group with five present
-    (100, 7, 130, 16),   # partial work-group, two chunks, seven columns
-    (300, 11, 258, 4),   # three chunks, 8 + 3 columns
-    (64, 13, 64, 0),     # nb < 128, 8 + 4 + 1 (the last column through the block dots)
-    (48, 64, 8, 0),      # the largest token count of the multi-column path
-    (40, 3, 7, 0),       # odd nb: the MFMA GEMM instead
+    (4096, 5, 128, 0),
+    (100, 7, 130, 16),   # 130 blocks: a chunk of two after whole ones
+    (300, 11, 258, 4),
+    (64, 13, 64, 0),
+    (48, 64, 8, 0),
+    (40, 3, 7, 0),       # odd nb
 ])
 def test_q8_0_gemm_few_tokens(hip, oracle, dev, nr, nc, nb, ypad):
-    """The a9 GEMM with a few tokens runs as GEMVs over groups of up to eight
-    activation columns: every output equals the oracle's (the a5 fold with the
-    exact d_x*d_y), and the output row padding stays untouched."""
+    """The a9 GEMM with a few tokens (two to four as one multi-column GEMV, more on 16 x 16 MFMA
+    tiles): every output equals the oracle's (the a5 fold with the exact d_x*d_y), and the output
+    row padding stays untouched."""
     n = nb * 32
     w = synth.q8_0_matrix(nr, n, 1015, 0.02)
     a = np.pad(synth.q8_0_matrix(nc, n, 1014, 1.0), ((0, 0), (0, ypad)))
@@ -432,13 +433,13 @@ def test_q8_0_gemm_few_tokens(hip, oracle, dev, nr, nc, nb, ypad):
     (1, 300, 64, 0, 8),       # single weight row: register-direct block dots
     (1, 33, 260, 0, 0),       # single weight row, 2 chunks + 4 blocks
     (512, 512, 128, 0, 0),
-    # 256+ weight rows take the wide 256x128 tile with 4-block K chunks
-    (300, 130, 7, 16, 32),    # partial wide tiles both ways, 4 + 3 blocks, padded strides
-    (256, 2, 1, 0, 0),        # one block: only the partial chunk
-    (520, 257, 13, 0, 4),     # three tile rows, 3 full chunks + 1 block
-    (300, 130, 8, 0, 0),      # two full chunks, partial tiles both ways
-    (520, 257, 16, 16, 32),   # four full chunks, padded strides, three tile rows
-    (256, 64, 8, 4, 0),       # one full tile row, a stride of 276 bytes
+    # (the 256-row tiles have theirs in test_gpu_reach.py)
+    (300, 130, 7, 16, 32),    # padded strides
+    (256, 2, 1, 0, 0),        # one block
+    (520, 257, 13, 0, 4),
+    (300, 130, 8, 0, 0),
+    (520, 257, 16, 16, 32),
+    (256, 64, 8, 4, 0),       # a stride of 276 bytes
 ])
 def test_q8_0_gemm(hip, oracle, dev, nr, nc, nb, xpad, ypad):
     n = nb * 32
@@ -1001,9 +1002,8 @@ def test_q8_0_gemm_tiles_and_ws(hip, oracle, dev, nr, nc, nb, xpad, ypad):
 
 @pytest.mark.parametrize("nb", [12, 13, 5])
 def test_q8_0_gemm_tiles_more_tiles_than_cus(hip, oracle, dev, nb):
-    """17 x 17 = 289 work-group tiles of the tiled kernel, partial ones on both
-    edges: more tiles than the part has CUs, so a second round of work-groups
-    runs.  K with no partial chunk (12 blocks), with one (13) and with only one
+    """4196 x 2118 outputs, 289 tiles of 256 x 128, partial ones on both edges: more than the part has
+    CUs, so the 192 x 256 tiles run.  K with no partial chunk (12 blocks), with one (13) and with only one
     (5).  The whole output equals the plain entry's bit for bit; sampled rows
     match the oracle."""
     nr, nc, n = 16 * 256 + 100, 16 * 128 + 70, nb * 32
@@ -1026,10 +1026,6 @@ def test_q8_0_gemm_tiles_more_tiles_than_cus(hip, oracle, dev, nb):
         assert_f32_parity(got[r, :nc], row, what=f"row {r}")
 
 
-def _rounds(nr, nc, bm, bn, cus=256):
-    return -(-(-(-nr // bm) * -(-nc // bn)) // cus)
-
-
 @pytest.mark.parametrize("nr,nc,nb,xpad,ypad", [
     (4096, 4096, 4, 0, 0),     # exactly one 4-block chunk: no DMA issued inside the fold
     (4096, 4096, 5, 0, 0),     # one chunk + 1: chunk 0's fold issues only block 0's slots
@@ -1045,7 +1041,9 @@ def test_q8_0_gemm_tiles_256x256(hip, oracle, dev, nr, nc, nb, xpad, ypad):
     equal the plain entry (another kernel, the same fold order) bit for bit over the whole
     output, the padding columns stay untouched, and sampled rows, the last included, match
     the oracle."""
-    assert _rounds(nr, nc, 256, 256) * 15 <= _rounds(nr, nc, 256, 128) * 8
+    runs = launches.kernels([launches.gemm_call("q8_0", e, nr, nc, nb * 32, xpad, ypad)
+                             for e in ("tiles", "ws")])
+    assert [names[-1] for names in runs] == ["gemm_tiles256_q8<Wave2x4>"] * 2
     n = nb * 32
     w = np.pad(synth.q8_0_matrix(nr, n, 1041, 0.02), ((0, 0), (0, xpad)))
     a = np.pad(synth.q8_0_matrix(nc, n, 1042, 1.0), ((0, 0), (0, ypad)))
@@ -1096,7 +1094,9 @@ def test_q4_0_gemm_tiles_256x256(hip, oracle, dev, nr, nc, nb, xpad, ypad):
     LDS): the pre-packed entry and the workspace entry equal the plain Q4_0 entry (another
     kernel, the same fold) bit for bit over the whole output, padding columns untouched,
     sampled rows, the last included, against the oracle."""
-    assert _rounds(nr, nc, 256, 256) * 15 <= _rounds(nr, nc, 256, 128) * 8
+    runs = launches.kernels([launches.gemm_call("q4_0", e, nr, nc, nb * 32, xpad, ypad)
+                             for e in ("tiles", "ws")])
+    assert [names[-1] for names in runs] == ["gemm_tiles256_q4<Wave2x4>"] * 2
     n = nb * 32
     w = np.pad(synth.q4_0_matrix(nr, n, 1043, 0.02), ((0, 0), (0, xpad)))
     a = np.pad(synth.q8_0_matrix(nc, n, 1044, 1.0), ((0, 0), (0, ypad)))
@@ -1209,8 +1209,8 @@ def test_gemm_tiles_one_tile_a_wave(hip, oracle, dev, quant, nr, nc, nb):
 ])
 def test_gemm_plain_rows_few_tiles(hip, oracle, dev, quant, nr, nc, nb):
     """The plain entries at shapes of few output tiles with 16-byte aligned rows and whole
-    8-block chunks: each work-group packs its 64 weight rows and 64 tokens into LDS records
-    chunk by chunk and folds one 32 x 32 tile a wave.  Whole outputs against the pre-packed
+    8-block chunks (gemm_rows_few, and gemm_rows16 and gemm_batch, which took most of them over).
+    Whole outputs against the pre-packed
     entry (the one-tile-a-wave kernels over the records) bit for bit, sampled rows against the
     oracle, with -128 block sums and a padded output stride."""
     n = nb * 32
@@ -1242,36 +1242,16 @@ def test_gemm_plain_rows_few_tiles(hip, oracle, dev, quant, nr, nc, nb):
         assert_f32_parity(got[r, :nc], row, what=f"{what}, row {r}")
 
 
-def _ws_route(nr, nc, nb, bx, by):
-    """Which kernel the workspace entries run (the host's rules, restated): the plain entry's
-    multi-column GEMVs for a few tokens, one tile a wave below one round of 256 x 128 tiles (and
-    at most 1024 of its 64 x 64 work-groups) -- 16 x 16 while those waves fit one a SIMD, the
-    plain entry's (packed in LDS) for 16-byte rows up to 448 work-groups and K 4096, else
-    32 x 32 -- else the 256 x 256 or 256 x 128 tiles by the rounds rule."""
-    if nc <= 24 and nb % 2 == 0 and bx % 4 == 0 and by % 4 == 0:
-        return "cols"
-    t64 = -(-nr // 64) * -(-nc // 64)
-    if -(-nr // 256) * -(-nc // 128) < 256 and t64 <= 1024:
-        if -(-nr // 32) * -(-nc // 32) <= 256:
-            return "16x16"
-        if nb % 8 == 0 and nb <= 128 and bx % 16 == 0 and by % 16 == 0 and t64 <= 448:
-            return "plain few tiles"
-        return "32x32"
-    return "256x256" if _rounds(nr, nc, 256, 256) * 15 <= _rounds(nr, nc, 256, 128) * 8 \
-        else "256x128"
-
-
 @pytest.mark.parametrize("quant", ["q8_0", "q4_0"])
 def test_gemm_ws_random_shapes(hip, oracle, dev, quant):
     """28 seeded random shapes through the workspace entry -- a few tokens, a few hundred,
-    thousands, and large outputs, so every route runs (the multi-column GEMVs, the one-tile-a-wave
-    kernel, both work-group tiles by the rounds rule) with every chunk and tail split -- against
+    thousands, and large outputs, so that the plain-row kernels of few outputs, one tile a wave and
+    the work-group tiles run, with every chunk and tail split -- against
     the plain entry, whole outputs bit for bit, with padded row strides and output strides; one
     sampled row of each against the oracle."""
     rng = np.random.default_rng(2026 if quant == "q8_0" else 2027)
     make = synth.q8_0_matrix if quant == "q8_0" else synth.q4_0_matrix
-    wb = 34 if quant == "q8_0" else 18
-    seen = set()
+    calls = []
     for case in range(28):
         kind = case % 4
         if kind == 3:
@@ -1283,7 +1263,7 @@ def test_gemm_ws_random_shapes(hip, oracle, dev, quant):
         n = nb * 32
         xpad, ypad = 2 * int(rng.integers(0, 9)), 2 * int(rng.integers(0, 9))
         bs = nc + int(rng.integers(0, 5))
-        seen.add(_ws_route(nr, nc, nb, nb * wb + xpad, nb * 34 + ypad))
+        calls.append(launches.gemm_call(quant, "ws", nr, nc, n, xpad, ypad))
         w = np.pad(make(nr, n, 3000 + case, 0.02), ((0, 0), (0, xpad)))
         a = np.pad(synth.q8_0_matrix(nc, n, 4000 + case, 1.0), ((0, 0), (0, ypad)))
         dw, da = to_dev(w, dev), to_dev(a, dev)
@@ -1305,7 +1285,11 @@ def test_gemm_ws_random_shapes(hip, oracle, dev, quant):
         row = ora(n, w[r].copy(), a, a.shape[1], 1, nc, w.shape[1], nc, 8)
         assert_f32_parity(got[r, :nc], row, what=f"{what}, row {r}")
         del dw, da, ref, ws, s
-    assert seen >= {"cols", "16x16", "32x32", "256x256", "256x128"}  # every route ran
+    # what ran, by the library's own rules (the other kernels: test_gpu_reach.py)
+    tag, k = ("true" if quant == "q4_0" else "false"), quant[:2]
+    assert {names[-1] for names in launches.kernels(calls)} >= {
+        f"gemm_batch<{tag}, 8, false>", f"gemm_rows16<{tag}, 2>", f"gemm_tiles32<{tag}>",
+        f"gemm_tiles256_{k}<Wave2x4>", f"gemm_tiles256_{k}<Wave3x2>"}
 
 
 def test_q8_0_gemm_ws_full_size_sampled(hip, oracle, dev):

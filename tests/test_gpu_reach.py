@@ -33,16 +33,19 @@ SIZES += both("gemm_batch<%, 16, false>", "plain", 300, 15, 67, 2, 0)
 SIZES += both("gemm_rows16<%, 2>", "plain", 2100, 66, 33, 0, 2)
 SIZES += both("gemm_rows16<%, 4>", "plain", 2100, 130, 22, 2, 0)
 SIZES += both("gemm_rows_few<%>", "plain", 1000, 800, 24, 0, 16)
-SIZES += both("gemm_wide<%>", "plain", 2100, 1000, 10, 0, 4)
+for nb, ypad in ((2, 0), (8, 4), (10, 4)):  # 4-block chunks: none, two whole, a part one
+    SIZES += both("gemm_wide<%>", "plain", 2100, 1000, nb, 0, ypad)
 SIZES += both("gemm_wide<%>", "plain", 2100, 1000, 42, 4, 0)
-SIZES += [("gemm_occ<true>", "q4_0", "plain", 200, 6190, 10, 0, 0),
-          ("gemm_occ<false>", "q8_0", "plain", 200, 5930, 10, 4, 0)]
+for nb, xpad in ((2, 0), (8, 4), (10, 0)):
+    SIZES += [("gemm_occ<true>", "q4_0", "plain", 200, 6190, nb, xpad, 0),
+              ("gemm_occ<false>", "q8_0", "plain", 200, 5930, nb, xpad, 0)]
 SIZES += both("gemm_tiles16<%>", "tiles", 300, 200, 9, 0, 0)
 SIZES += both("gemm_tiles32<%>", "tiles", 1000, 700, 9, 0, 0)
 for q in ("q4_0", "q8_0"):
-    SIZES += [("gemm_tiles_q4" if q == "q4_0" else "gemm_tiles_q8<true>", q, "tiles", 3100, 2100, 13,
-               0, 0),
-              (f"gemm_tiles256_{q[:2]}<Wave2x4>", q, "tiles", 3400, 3700, 13, 0, 0),
+    for nb in (5, 6, 13):  # 6-block chunks: none, one whole, a part one
+        SIZES.append(("gemm_tiles_q4" if q == "q4_0" else "gemm_tiles_q8<true>", q, "tiles", 3100,
+                      2100, nb, 0, 0))
+    SIZES += [(f"gemm_tiles256_{q[:2]}<Wave2x4>", q, "tiles", 3400, 3700, 13, 0, 0),
               (f"gemm_tiles256_{q[:2]}<Wave3x2>", q, "tiles", 4000, 2900, 13, 0, 0)]
 # x16 weights: weight rows a multiple of 16, tokens of 4; the pad is of the output rows
 SIZES += [("gemm_repack_q4_0", "q4_0", "repack", 2064, 2052, 9, 0, 0),

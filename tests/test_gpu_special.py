@@ -57,16 +57,17 @@ def q4(rows, nb, seed, nonfinite_every=0):
 # ------------------------------------------------------------------ GEMMs ---
 
 @pytest.mark.parametrize("nr,nc,nb,pad", [
-    (300, 130, 9, 0),    # wide 256 x 128 tiles: 2 full chunks + 1 block
-    (256, 128, 8, 0),    # few tiles, 16-byte rows: packed in LDS, one 32 x 32 tile a wave
-    (600, 200, 24, 0),   # the same over three 8-block chunks
-    (600, 200, 48, 0),   # the same over six chunks
-    (100, 70, 9, 16),    # 128 x 128 tiles (fewer than 256 weight rows)
-    (33, 20, 5, 2),      # rows 2-byte aligned only: the raw-block kernel
+    # nc > 1: gemm_batch (the other GEMM kernels: test_gpu_reach.py)
+    (300, 130, 9, 0),
+    (256, 128, 8, 0),
+    (600, 200, 24, 0),
+    (600, 200, 48, 0),
+    (100, 70, 9, 16),
+    (33, 20, 5, 2),      # rows 2-byte aligned only
     (64, 1, 8, 0),       # decode shape: register-direct block dots
     (1, 40, 8, 0),       # one weight row
-    (200, 6, 8, 0),      # a few tokens: the multi-column GEMV (8 columns, six present)
-    (64, 3, 10, 0),      # a few tokens: 4 columns, three present
+    (200, 6, 8, 0),
+    (64, 3, 10, 0),
 ])
 def test_q8_0_gemm_special_scales(hip, oracle, dev, nr, nc, nb, pad):
     n = nb * 32
@@ -79,7 +80,7 @@ def test_q8_0_gemm_special_scales(hip, oracle, dev, nr, nc, nb, pad):
 
 
 def test_q8_0_gemm_ws_special_scales(hip, oracle, dev):
-    """The workspace entry at a shape of few tiles (its one-tile-a-wave kernel)."""
+    """The workspace entry at a shape of few outputs (gemm_batch over the plain rows)."""
     nr, nc, nb = 300, 130, 9
     n = nb * 32
     w = q8(nr, nb, 31, 0.02, nonfinite_every=16)
@@ -94,9 +95,7 @@ def test_q8_0_gemm_ws_special_scales(hip, oracle, dev):
 
 
 @pytest.mark.parametrize("nr,nc,nb", [(300, 130, 9), (100, 70, 9), (64, 1, 8), (1, 40, 8),
-                                      (600, 200, 24),  # packed in LDS, a 32 x 32 tile a wave
-                                      (600, 200, 48),  # the same, six chunks
-                                      (200, 4, 8), (64, 3, 10)])  # the last two: multi-column GEMVs
+                                      (600, 200, 24), (600, 200, 48), (200, 4, 8), (64, 3, 10)])
 def test_q4_0_gemm_special_scales(hip, oracle, dev, nr, nc, nb):
     n = nb * 32
     w = q4(nr, nb, 13, nonfinite_every=16)
@@ -108,7 +107,7 @@ def test_q4_0_gemm_special_scales(hip, oracle, dev, nr, nc, nb):
 
 
 def test_q4_0_gemm_tiles_special_scales(hip, oracle, dev):
-    """The tiled Q4_0 GEMM over the GEMM-tile layout at a shape of few tiles (one 32 x 32 tile
+    """The tiled Q4_0 GEMM over the GEMM-tile layout at a shape of few tiles (one 16 x 16 tile
     a wave)."""
     nr, nc, nb = 300, 130, 9
     n = nb * 32
@@ -120,9 +119,8 @@ def test_q4_0_gemm_tiles_special_scales(hip, oracle, dev):
 
 
 def test_q4_0_gemm_ws_special_scales(hip, oracle, dev):
-    """The workspace entry: both operands packed in one launch (16-byte aligned
-    rows, 8-block spans), then the tiled Q4_0 GEMM (one 32 x 32 tile a wave at
-    this shape)."""
+    """The workspace entry with 16-byte aligned rows at a shape of few outputs (gemm_batch over the
+    plain rows)."""
     nr, nc, nb = 320, 96, 16
     n = nb * 32
     w = q4(nr, nb, 35, nonfinite_every=16)
@@ -142,7 +140,7 @@ def test_q4_0_gemm_tiles_nonfinite_dx_mid_k(hip, oracle, dev):
     across K: +-Inf planted in the first blocks, in the middle of K and near its
     end, NaN, and an infinite d_x over a zero block sum (0 * Inf = NaN).  The
     256-row tiles' fast-to-exact switch is covered by
-    test_gemm_ws_tiles_special_scales."""
+    test_gemm_ws_tiles_special_scales and test_gpu_reach.py."""
     nr, nc, nb = 512, 256, 40  # 6 full chunks + 4 tail blocks
     n = nb * 32
     w = q4(nr, nb, 41)
@@ -161,11 +159,10 @@ def test_q4_0_gemm_tiles_nonfinite_dx_mid_k(hip, oracle, dev):
 
 @pytest.mark.parametrize("nb", [40, 42])
 def test_q4_0_gemm_nonfinite_dx_mid_k(hip, oracle, dev, nb):
-    """The plain Q4_0 entry with non-finite d_x planted across K (nb = 40: the
-    plain-row few-tile kernel, one 32 x 32 tile a wave; nb = 42: the 256 x 128
-    wide kernel): +-Inf in the first chunk of one wave's rows, in the middle of K,
-    in the last block and (nb = 42) in the partial tail, NaN, and an infinite
-    d_x over a zero block sum (0 * Inf = NaN)."""
+    """The plain Q4_0 entry with non-finite d_x planted across K (gemm_batch; the 256 x 128 wide
+    kernel, whose fold switches form in the middle of K: test_gpu_reach.py): +-Inf in the first
+    blocks, in the middle of K and in the last block, NaN, and an infinite d_x over a zero block
+    sum (0 * Inf = NaN)."""
     nr, nc = 512, 256
     n = nb * 32
     w = q4(nr, nb, 43)
@@ -183,14 +180,13 @@ def test_q4_0_gemm_nonfinite_dx_mid_k(hip, oracle, dev, nb):
     assert np.isinf(g[70]).any() and np.isnan(g[400]).all()  # the planted cases took effect
 
 
-@pytest.mark.parametrize("nr,nc,kernel", [(4096, 4096, "256x256"), (4196, 4166, "256x128"),
-                                          (4096, 130, "32x32"), (4096, 40, "16x16")])
+@pytest.mark.parametrize("nr,nc,kernel", [(4096, 4096, "256x256"), (4196, 4166, "192x256"),
+                                          (4096, 130, "32x32"), (4096, 40, "plain rows")])
 @pytest.mark.parametrize("quant,nonfinite_every", [("q8_0", 16), ("q4_0", 16), ("q4_0", 0)])
 def test_gemm_ws_tiles_special_scales(hip, oracle, dev, quant, nonfinite_every, nr, nc, kernel):
-    """Each work-group tile of the tiled GEMMs, through the workspace entries (256 x 256: 4096 x
-    4096 outputs; 256 x 128: 4196 x 4166, three rounds of it against two of the larger tile; one
-    32 x 32 tile a wave: 4096 x 130; one 16 x 16 tile a wave: 4096 x 40): special scales in both
-    operands, non-finite d_x in every
+    """The workspace entries' kernels (256 x 256 tiles: 4096 x 4096 outputs; 192 x 256: 4196 x 4166;
+    one 32 x 32 tile a wave: 4096 x 130; gemm_rows16 over the plain rows: 4096 x 40; the others:
+    test_gpu_reach.py): special scales in both operands, non-finite d_x in every
     16th weight row (every Q4_0 wave of the 256-row tiles folds exactly from chunk 0) or, with
     none there, +-Inf and NaN planted at chunk 0, in the middle of K, in the last full chunk and
     in the 1-block tail (chunks of 4 and of 6 blocks), and an infinite d_x over a zero block
