@@ -44,10 +44,10 @@ def test_kernel_of_a_size(size):
 
 
 @pytest.mark.parametrize("quant,nr,nc,n,want", [
-    ("q4_0", 15568, 33, 6656, "pack_tiles_ranges2<true, 2>"),
-    ("q8_0", 4096, 4096, 4096, "pack_tiles_ranges2<false, 2>"),  # 1024 ranges of weights
-    ("q8_0", 4032, 4096, 4096, "pack_tiles_ranges2<false, 1>"),  # 1008
-    ("q8_0", 3001, 4096, 2912, "pack_tiles_ranges2<false, 1>"),
+    ("q4_0", 15568, 33, 6656, "pack_tiles_ranges2<true, 2, true>"),
+    ("q8_0", 4096, 4096, 4096, "pack_tiles_ranges2<false, 2, false>"),  # 1024 ranges of weights
+    ("q8_0", 4032, 4096, 4096, "pack_tiles_ranges2<false, 1, false>"),  # 1008
+    ("q8_0", 3001, 4096, 2912, "pack_tiles_ranges2<false, 1, false>"),
 ])
 def test_pack_of_a_workspace_gemm(quant, nr, nc, n, want):
     assert launches.kernels([launches.gemm_call(quant, "ws", nr, nc, n)])[0][0] == want

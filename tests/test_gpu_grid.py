@@ -10,6 +10,7 @@ from gpu_util import assert_f32_parity, assert_f32_parity_nan, from_dev, to_dev
 
 GRID = "block_dot_pairs<(DotFmt)1, false, true>"
 BATCH8, BATCH16 = "gemm_batch<true, 8, false>", "gemm_batch<true, 16, false>"
+ONE8, ONE16 = "gemm_batch_one<true, 8>", "gemm_batch_one<true, 16>"
 
 SIZES = [
     # nr, nc, nb, weight pad, token pad, offset, kernel
@@ -22,15 +23,15 @@ SIZES = [
     (64, 32, 128, 2, 2, 0, GRID),      # one whole chunk, 2048 outputs
     (64, 33, 128, 2, 2, 0, BATCH16),   # 2112, 176 a tile
     (832, 4, 129, 0, 0, 0, GRID),      # 3328, 64 a tile
-    (1665, 2, 129, 0, 0, 0, BATCH8),
-    (560, 5, 129, 0, 0, 0, BATCH8),    # 2800, 80 a tile
+    (1665, 2, 129, 0, 0, 0, ONE8),
+    (560, 5, 129, 0, 0, 0, ONE8),    # 2800, 80 a tile
     (5, 3, 257, 0, 4, 2, GRID),        # a chunk of one block
     (200, 20, 131, 0, 0, 2, BATCH8),   # three 8-wave chunks, the last of three blocks
-    (1700, 2, 257, 0, 4, 0, BATCH8),   # five chunks, one block in the last
-    (520, 7, 65, 0, 0, 0, BATCH16),    # 16 waves, nine of them with blocks
-    (400, 7, 63, 2, 6, 2, BATCH8),     # every slice, the last one block short
-    (2, 2, 8, 2, 2, 0, BATCH8),
-    (4, 3, 64, 0, 0, 0, BATCH8),       # 4-byte aligned rows: the rule is not for them
+    (1700, 2, 257, 0, 4, 0, ONE8),   # five chunks, one block in the last
+    (520, 7, 65, 0, 0, 0, ONE16),    # 16 waves, nine of them with blocks
+    (400, 7, 63, 2, 6, 2, ONE8),     # every slice, the last one block short
+    (2, 2, 8, 2, 2, 0, ONE8),
+    (4, 3, 64, 0, 0, 0, ONE8),       # 4-byte aligned rows: the rule is not for them
 ]
 
 

@@ -1288,7 +1288,7 @@ def test_gemm_ws_random_shapes(hip, oracle, dev, quant):
     # what ran, by the library's own rules (the other kernels: test_gpu_reach.py)
     tag, k = ("true" if quant == "q4_0" else "false"), quant[:2]
     assert {names[-1] for names in launches.kernels(calls)} >= {
-        f"gemm_batch<{tag}, 8, false>", f"gemm_rows16<{tag}, 2>", f"gemm_tiles32<{tag}>",
+        f"gemm_batch_one<{tag}, 8>", f"gemm_rows16<{tag}, 2>", f"gemm_tiles32<{tag}>",
         f"gemm_tiles256_{k}<Wave2x4>", f"gemm_tiles256_{k}<Wave3x2>"}
 
 

@@ -28,8 +28,10 @@ SIZES = [s for quant in ("q4_0", "q8_0") for s in [
     (f"gemv_{quant}_q8_0_cols<4, true>", quant, "plain", 37, 3, 128, 0, 0),
     (f"gemv_{quant}_q8_0_cols<4, false>", quant, "plain", 37, 4, 258, 0, 4),
 ]]
-SIZES += both("gemm_batch<%, 8, false>", "plain", 300, 15, 67 + 64, 0, 0)
-SIZES += both("gemm_batch<%, 16, false>", "plain", 300, 15, 67, 2, 0)
+SIZES += both("gemm_batch<%, 8, false>", "plain", 300, 30, 67 + 64, 0, 0)
+SIZES += both("gemm_batch<%, 16, false>", "plain", 300, 30, 67, 2, 0)
+SIZES += both("gemm_batch_one<%, 8>", "plain", 300, 15, 67 + 64, 0, 0)
+SIZES += both("gemm_batch_one<%, 16>", "plain", 300, 15, 67, 2, 0)
 SIZES += both("gemm_rows16<%, 2>", "plain", 2100, 66, 33, 0, 2)
 SIZES += both("gemm_rows16<%, 4>", "plain", 2100, 130, 22, 2, 0)
 SIZES += both("gemm_rows_few<%>", "plain", 1000, 800, 24, 0, 16)

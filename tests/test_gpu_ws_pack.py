@@ -24,7 +24,8 @@ SIZES = [
 def test_launch(quant, nr, nc, nb, xpad, ypad, each, group_wgs):
     (status, xs), = launches.replay([launches.gemm_call(quant, "ws", nr, nc, nb * 32, xpad, ypad)])
     assert status == 0
-    assert xs[0].name == f"pack_tiles_ranges2<{'true' if quant == 'q4_0' else 'false'}, {each}>"
+    assert xs[0].name == (f"pack_tiles_ranges2<{'true' if quant == 'q4_0' else 'false'}, {each}, "
+                          f"{'true' if group_wgs else 'false'}>")
     groups, ranges = -(-nr // 64), -(-nb // 8)
     xgrid = -(-groups // 8) * 8 * group_wgs if group_wgs else -(-groups * ranges // each)
     assert xs[0].grid == (xgrid + -(-nc // 64) * ranges, 1, 1)

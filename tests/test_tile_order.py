@@ -61,7 +61,8 @@ def test_every_tile_once_and_balanced(tmp_path):
 
 
 # the row and token extent of a work-group's tile
-TILES = {"gemm_batch": lambda a: (16, 16), "gemm_rows16": lambda a: (16 * int(a[1]), 32),
+TILES = {"gemm_batch": lambda a: (16, 16), "gemm_batch_one": lambda a: (16, 16),
+         "gemm_rows16": lambda a: (16 * int(a[1]), 32),
          "gemm_repack_mid": lambda a: (32 * int(a[0]), 32 * int(a[1]))}
 
 
@@ -72,7 +73,8 @@ TILES = {"gemm_batch": lambda a: (16, 16), "gemm_rows16": lambda a: (16 * int(a[
     ("q8_0", "ws", 1170, 327, 12608, "gemm_rows16"),
     ("q4_0", "plain", 16, 4096, 4096, "gemm_batch"),    # one row tile, 256 token groups
     ("q8_0", "plain", 2, 319, 12064, "gemm_batch"),
-    ("q4_0", "plain", 4096, 16, 4096, "gemm_batch"),
+    ("q4_0", "plain", 4096, 16, 4096, "gemm_batch_one"),
+    ("q8_0", "plain", 4100, 2, 2912, "gemm_batch_one"),
     ("q4_0", "repack", 2176, 768, 4096, "gemm_repack_mid"),  # 17 x 12
     ("q4_0", "repack", 512, 4096, 4096, "gemm_repack_mid"),
     ("q4_0", "repack", 1152, 1088, 4096, "gemm_repack_mid"),

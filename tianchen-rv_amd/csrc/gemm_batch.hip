@@ -107,14 +107,12 @@ __device__ __forceinline__ v4i bt_sums(uint32_t a0, uint32_t a1, uint32_t b0, ui
   return __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, v4i{}, 0, 0, 0);
 }
 
-// Work-group (x, y, z): the tile of XCD x's slot (y, z), tile_order.h.  At
-// most four waves a SIMD: two work-groups of 8 waves a CU, one of 16.
-// kWide: row strides past 256 MB.
+// The tile of rows row0.. and tokens tok0..  At most four waves a SIMD (the kernels' bounds): two
+// work-groups of 8 waves a CU, one of 16.  kWide: row strides past 256 MB.
 template <bool kQ4, int kWaves, bool kWide>
-__global__ __launch_bounds__(kWaves * 64, 4) void gemm_batch(
-    uint32_t units, uint32_t inv, const uint8_t *vx,
-    size_t bx, const uint8_t *vy, size_t by, uint32_t nr, uint32_t nc, size_t nb, float *s,
-    size_t bs) {
+__device__ __forceinline__ void batch_tile(size_t row0, unsigned tok0, const uint8_t *vx, size_t bx,
+                                           const uint8_t *vy, size_t by, size_t nr, size_t nb,
+                                           unsigned nc, float *s, size_t bs) {
   using Off = std::conditional_t<kWide, size_t, uint32_t>;  // of a row from the tile's first
   constexpr int kChunk = kWaves * kBtSlice;  // blocks
   constexpr int kXBlock = kQ4 ? kQ4Bytes : kQ8Bytes;
@@ -131,13 +129,6 @@ __global__ __launch_bounds__(kWaves * 64, 4) void gemm_batch(
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
-  const TilePos tile = xcd_tile(units, (nr + kBtRows - 1) / kBtRows,
-                                (nc + kBtToks - 1) / kBtToks, inv, blockIdx.x, blockIdx.y,
-                                blockIdx.z);
-  if (!tile.live)
-    return;
-  const size_t row0 = static_cast<size_t>(tile.tm) * kBtRows;
-  const unsigned tok0 = tile.tn * kBtToks;
   const int ntok = static_cast<int>(min(nc - tok0, static_cast<unsigned>(kBtToks)));
   uint8_t *region = lds + wave * kBtRegion;
 
@@ -314,14 +305,38 @@ __global__ __launch_bounds__(kWaves * 64, 4) void gemm_batch(
     s[(row0 + fr) * bs + tok0 + li] = kQ4 ? acc * 0.0625f : acc;
 }
 
+// Work-group (x, y, z): the tile of XCD x's slot (y, z), tile_order.h.
+template <bool kQ4, int kWaves, bool kWide>
+__global__ __launch_bounds__(kWaves * 64, 4) void gemm_batch(
+    const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by, size_t nb, uint32_t nr, uint32_t nc,
+    uint32_t units, uint32_t inv, float *s, size_t bs) {
+  const TilePos tile = xcd_tile(units, (nr + kBtRows - 1) / kBtRows, (nc + kBtToks - 1) / kBtToks,
+                                inv, blockIdx.x, blockIdx.y, blockIdx.z);
+  if (tile.live)
+    batch_tile<kQ4, kWaves, kWide>(static_cast<size_t>(tile.tm) * kBtRows, tile.tn * kBtToks, vx, bx,
+                                   vy, by, nr, nb, nc, s, bs);
+}
+
+// One token group: the row tiles dealt in turn, which is as even and spares a wave the order's
+// arithmetic (1-2 % of a 4-7 us kernel).
+template <bool kQ4, int kWaves>
+__global__ __launch_bounds__(kWaves * 64, 4) void gemm_batch_one(
+    const uint8_t *vx, size_t bx, const uint8_t *vy, size_t by, size_t nr, size_t nb, unsigned nc,
+    float *s, size_t bs) {
+  const unsigned tile = blockIdx.x + kXcds * blockIdx.y;
+  const size_t row0 = static_cast<size_t>(tile) * kBtRows;
+  if (row0 < nr)
+    batch_tile<kQ4, kWaves, false>(row0, 0, vx, bx, vy, by, nr, nb, nc, s, bs);
+}
+
 }  // namespace tcrv
 
 namespace tcrv_host {
 
 int gemm_batch(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const uint8_t *vy,
                size_t by, size_t nr, size_t nc, size_t bs, void *stream) {
-  // a launch takes 2^19 row tiles, then as many token groups as its tiles allow
-  constexpr size_t kMaxRows = (static_cast<size_t>(1) << 19) * tcrv::kBtRows;
+  // a launch takes 65535 x 8 row tiles, then as many token groups as its tiles allow
+  constexpr size_t kMaxRows = static_cast<size_t>(65535) * 8 * tcrv::kBtRows;
   const bool wide = bx > 0x0fffffffu || by > 0x0fffffffu;
   hipStream_t st = as_stream(stream);
   for (size_t r0 = 0; r0 < nr; r0 += kMaxRows) {
@@ -331,28 +346,41 @@ int gemm_batch(bool q4, size_t nb, float *s, const uint8_t *vx, size_t bx, const
     for (size_t c0 = 0; c0 < nc; c0 += max_toks) {
       const size_t toks = nc - c0 < max_toks ? nc - c0 : max_toks;
       const size_t groups = (toks + tcrv::kBtToks - 1) / tcrv::kBtToks;
-      tcrv::TileOrder o;
-      if (!tcrv::tile_order(tiles, groups, &o))
-        return TCRV_HIP_ERR_TOO_LARGE;
-      const dim3 g(tcrv::kXcds, o.slots_y, o.slots_z);
-      auto run = [&](auto kernel, int waves) {
-        kernel<<<g, dim3(waves * 64), 0, st>>>(o.units, o.inv, vx + r0 * bx,
-                                               bx, vy + c0 * by, by, static_cast<uint32_t>(rows),
-                                               static_cast<uint32_t>(toks), nb,
-                                               s + r0 * bs + c0, bs);
-      };
+      const uint8_t *x = vx + r0 * bx, *y = vy + c0 * by;
+      float *out = s + r0 * bs + c0;
+      const uint32_t nt = static_cast<uint32_t>(toks);
       // 16 waves where they hold all of K in one chunk and 8 would not, and a CU
       // has one work-group at most (4096 x 16 x 4096 Q4_0 6.2 against 6.8 us,
       // Q8_0 7.0 against 8.0); with more work-groups two of 8 waves overlap
       // each other's loads (4096 x 32: 10.1 against 11.2; 4096 x 16 x 14336
       // 17.6 against 21.2)
       const bool w16 = nb > 64 && nb <= 128 && tiles * groups <= 256;
-      if (wide)
-        q4 ? run(tcrv::gemm_batch<true, 8, true>, 8) : run(tcrv::gemm_batch<false, 8, true>, 8);
-      else if (w16)
-        q4 ? run(tcrv::gemm_batch<true, 16, false>, 16) : run(tcrv::gemm_batch<false, 16, false>, 16);
-      else
-        q4 ? run(tcrv::gemm_batch<true, 8, false>, 8) : run(tcrv::gemm_batch<false, 8, false>, 8);
+      if (groups == 1 && !wide) {
+        auto run = [&](auto kernel, int waves) {
+          kernel<<<dim3(tcrv::kXcds, static_cast<unsigned>((tiles + 7) / 8)), dim3(waves * 64), 0,
+                   st>>>(x, bx, y, by, rows, nb, nt, out, bs);
+        };
+        if (w16)
+          q4 ? run(tcrv::gemm_batch_one<true, 16>, 16) : run(tcrv::gemm_batch_one<false, 16>, 16);
+        else
+          q4 ? run(tcrv::gemm_batch_one<true, 8>, 8) : run(tcrv::gemm_batch_one<false, 8>, 8);
+      } else {
+        tcrv::TileOrder o;
+        if (!tcrv::tile_order(tiles, groups, &o))
+          return TCRV_HIP_ERR_TOO_LARGE;
+        auto run = [&](auto kernel, int waves) {
+          kernel<<<dim3(tcrv::kXcds, o.slots_y, o.slots_z), dim3(waves * 64), 0, st>>>(
+              x, bx, y, by, nb, static_cast<uint32_t>(rows), nt, o.units, o.inv, out, bs);
+        };
+        if (wide)
+          q4 ? run(tcrv::gemm_batch<true, 8, true>, 8) : run(tcrv::gemm_batch<false, 8, true>, 8);
+        else if (w16)
+          q4 ? run(tcrv::gemm_batch<true, 16, false>, 16)
+             : run(tcrv::gemm_batch<false, 16, false>, 16);
+        else
+          q4 ? run(tcrv::gemm_batch<true, 8, false>, 8)
+             : run(tcrv::gemm_batch<false, 8, false>, 8);
+      }
       const int rc = launch_status();
       if (rc != TCRV_HIP_OK)
         return rc;

@@ -344,15 +344,15 @@ struct SpanOperand {
   uint8_t *dst;
 };
 
-// The first xgrid work-groups pack x: in order, or (group_wgs > 0, the work-groups of a row group)
-// row group g on XCD g % 8, where gemm_tiles32 reads it.
-template <bool kXQ4, int kXR>
-__global__ __launch_bounds__(256) void pack_tiles_ranges2(size_t nb, SpanOperand x, SpanOperand y,
-                                                          uint32_t xgrid, uint32_t group_wgs) {
+// The first xgrid work-groups pack x: in order, or (kByXcd; group_wgs are the work-groups of a row
+// group) row group g on XCD g % 8, where gemm_tiles32 reads it.
+template <bool kXQ4, int kXR, bool kByXcd>
+__global__ __launch_bounds__(256) void pack_tiles_ranges2(uint32_t xgrid, uint32_t group_wgs,
+                                                          size_t nb, SpanOperand x, SpanOperand y) {
   __shared__ __align__(16) uint8_t raw[kXR * kTG * kPackSpan * kQ8Bytes];
   if (blockIdx.x < xgrid) {
     size_t wg = blockIdx.x;
-    if (group_wgs != 0) {
+    if constexpr (kByXcd) {
       const uint32_t k = blockIdx.x / 8, turn = k / group_wgs;
       wg = (8 * static_cast<size_t>(turn) + blockIdx.x % 8) * group_wgs + (k - turn * group_wgs);
       if (wg * kXR >= x.nranges)
@@ -1719,13 +1719,20 @@ int pack_tiles_both(size_t nb, const uint8_t *vx, size_t bx, size_t nr, uint8_t 
     return TCRV_HIP_ERR_TOO_LARGE;
   const dim3 g(static_cast<unsigned>(grid)), b(256);
   auto run = [&](auto kernel) {
-    kernel<<<g, b, 0, st>>>(nb, x, y, static_cast<uint32_t>(xgrid),
-                            static_cast<uint32_t>(group_wgs));
+    kernel<<<g, b, 0, st>>>(static_cast<uint32_t>(xgrid), static_cast<uint32_t>(group_wgs), nb, x, y);
   };
-  if (pairs)
-    xq4 ? run(tcrv::pack_tiles_ranges2<true, 2>) : run(tcrv::pack_tiles_ranges2<false, 2>);
+  if (group_wgs != 0 && pairs)
+    xq4 ? run(tcrv::pack_tiles_ranges2<true, 2, true>)
+        : run(tcrv::pack_tiles_ranges2<false, 2, true>);
+  else if (group_wgs != 0)
+    xq4 ? run(tcrv::pack_tiles_ranges2<true, 1, true>)
+        : run(tcrv::pack_tiles_ranges2<false, 1, true>);
+  else if (pairs)
+    xq4 ? run(tcrv::pack_tiles_ranges2<true, 2, false>)
+        : run(tcrv::pack_tiles_ranges2<false, 2, false>);
   else
-    xq4 ? run(tcrv::pack_tiles_ranges2<true, 1>) : run(tcrv::pack_tiles_ranges2<false, 1>);
+    xq4 ? run(tcrv::pack_tiles_ranges2<true, 1, false>)
+        : run(tcrv::pack_tiles_ranges2<false, 1, false>);
   return launch_status();
 }
 
